@@ -14,9 +14,11 @@
 //            macros, then S1 of the next step (gBarPvol = (1-r) g~ + r geq), written to the other
 //            ping-pong buffer.
 //
-// No per-(face, velocity) array exists: face values are recomputed from the resident state where
-// they are needed, so a step streams the distributions through HBM three times (two reads, one
-// write) and the neighbour rows of the gradients come from L2.
+// Here no per-(face, velocity) array exists: face values are recomputed from the resident state
+// where they are needed, so a step streams the distributions through HBM three times (two reads, one
+// write) and the neighbour rows of the gradients come from L2.  Where there is memory for them the
+// face values are stored instead (face-value mode), and meshes of cells with few faces then take the
+// kernels over velocity columns of lines.h, with the row order that goes with them.
 //
 // Data layout: distributions are [cell][velocity] with the velocity index contiguous and padded to
 // NVP = NT*NITER; a workgroup's lanes are velocities of one cell or face, so every mesh quantity is
@@ -46,7 +48,9 @@
 #include <cstring>
 #include <mutex>
 #include <new>
+#include <numeric>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/dugks.h"
@@ -178,7 +182,8 @@ struct alignas(64) CellSt {
     double a[MAXS];       // wall entries: 1/deltaCoeffs
     int32_t wmask;        // bit j set: entry j is a wall face
     int32_t inner;        // 1: every slot is an internal face (KIND_OWN or KIND_NEI)
-    int32_t pad[14];
+    int32_t plain;        // 1: S7 relaxes every value of every face (internal and cyclic faces only)
+    int32_t pad[13];
 };
 static_assert(sizeof(CellSt) % 64 == 0, "cellst size");
 
@@ -192,6 +197,25 @@ struct alignas(16) FaceX {
     int32_t kind, bidx;  // KIND_OWN (internal), KIND_WALL, KIND_CYC; wall index
 };
 static_assert(sizeof(FaceX) == 96, "facex size");
+
+struct LineRec;   // lines.h
+struct LineCell;  // lines.h
+
+// What the column form of k_cell needs of a (cell, face) slot in every iteration: the face
+// equilibrium along the loop axis, 1 - r, and +-S dt / V of that axis.  Written by k_face_fin.
+struct alignas(64) LineFace {
+    double invRT, B, qz, omr, Sl, RT, pad[2];
+};
+
+// Geometry of a (cell, face) slot for the column kernels: centre to face, and the outward area
+// vector, its loop-axis component apart.  NS entries per cell; those past its faces have S = 0 and
+// the cell's first face.
+struct alignas(64) LineGeo {
+    double dC[3];
+    double S[2], Sl, pad;
+    int32_t face, kind;
+};
+static_assert(sizeof(LineGeo) == 64, "linegeo size");
 
 template <typename TS>
 struct P {
@@ -232,6 +256,16 @@ struct P {
     const int *__restrict__ open;  // their face indices
     const int *__restrict__ fsel;  // k_face_moments over a face list (the wall faces), else null
     int nfsel;
+    // velocity columns (lines.h): the lanes of each tile, the iterations before each tile; moment records of the (cell, face) slots and of the open faces' incoming halves; per
+    // face {owner slot, neighbour slot or -1, open index or -1, 0}
+    const LineRec *__restrict__ rec;
+    const int *__restrict__ titer;
+    const LineGeo *__restrict__ lgeo;
+    int ntile, ntl;                 // tiles; tiles whose new row k_cell_lines keeps in LDS
+    double *spart, *opart;
+    LineFace *lface;
+    LineCell *lcell;
+    const int4 *__restrict__ fslot;
     const int *__restrict__ mxf;   // k_face_moments_mx: non-wall faces in launch order, 16 per tile (-1 pads)
     int *flag;
 };
@@ -254,6 +288,8 @@ DEVI double dotnc(double ax, double ay, double az, const double *b)
     return (ax * b[0] + ay * b[1]) + az * b[2];
 }
 
+constexpr size_t LDS_CU = 160 * 1024;   // LDS of a compute unit
+constexpr int NCU = 256;   // compute units of an MI355X
 constexpr int NXCD = 8;  // accelerator complex dies of an MI355X, each with its own L2
 
 template <typename TS>
@@ -659,11 +695,11 @@ DEVI bool need_N(int kind, double s)
 // least-squares gradients read are then shared through that XCD's L2.  Returns false for the
 // padding workgroups.
 // ---------------------------------------------------------------------------------------------
-DEVI bool xcd_block(int n, int nb, int &pos, int &b)
+DEVI bool xcd_block(int n, int nb, int &pos, int &b, int first = 0)
 {
-    const int per = (n + NXCD - 1) / NXCD;
+    const int per = (n + NXCD - 1) / NXCD, x = (int)blockIdx.x - first;
     b = (int)blockIdx.y;
-    pos = (int)(blockIdx.x % NXCD) * per + (int)(blockIdx.x / NXCD);
+    pos = (x % NXCD) * per + x / NXCD;
     return pos < n && b < nb;
 }
 
@@ -926,14 +962,11 @@ __global__ __launch_bounds__(MAXNT) __attribute__((amdgpu_waves_per_eu(kfv_waves
 // Fixed (mixed, frozen at the initial boundary Maxwellian, discreteVelocity.C:312-344):
 // rho_b M(U_b, T_b).  h = g R T_b (K + 3 - D) for the Maxwellians.
 // ---------------------------------------------------------------------------------------------
-template <int D, bool H, int NS, typename TS>
-__global__ __launch_bounds__(MAXNT) void k_face_open(P<TS> p)
+// open_face: the velocities k0, k0 + step, ... below k1 of open face i.  MOM: also adds the moments
+// of the values it writes, about the owner cell's velocity, to acc.
+template <int D, bool H, int NS, bool MOM, typename TS>
+DEVI void open_face(const P<TS> &p, int i, unsigned k0, unsigned k1, unsigned step, const double *vt, double *acc)
 {
-    __shared__ double vt[VT_SIZE];
-    const int i = blockIdx.x, b = blockIdx.y;
-    if (i >= p.nopen || b >= p.nb) return;
-    stage_vt(p, vt);
-    __syncthreads();
     const int f = cptr(p.open)[i];
     const CONST_AS FaceX &fx = cptr(p.fx)[f];
     const int c = fx.P;
@@ -945,17 +978,17 @@ __global__ __launch_bounds__(MAXNT) void k_face_open(P<TS> p)
     const bool fixedU = W.mode == 1.0;
     const double Ui[3] = {fixedU ? W.U[0] : cptr(p.cU)[3 * c], fixedU ? W.U[1] : cptr(p.cU)[3 * c + 1],
                           fixedU ? W.U[2] : cptr(p.cU)[3 * c + 2]};
+    const double Uo[3] = {cptr(p.cU)[3 * c], cptr(p.cU)[3 * c + 1], cptr(p.cU)[3 * c + 2]};
     const double RT = p.R * W.T;
     const TS *__restrict__ rowC = p.gb_in + (size_t)c * p.nvp;
     const TS *__restrict__ hrowC = H ? p.hb_in + (size_t)c * p.nvp : nullptr;
     TS *__restrict__ fg = p.fvg + (size_t)f * p.nvp;
     TS *__restrict__ fh = H ? p.fvh + (size_t)f * p.nvp : nullptr;
-    const unsigned k0 = (unsigned)b * p.vb + threadIdx.x;
-    for (int it = 0; it < p.nib; ++it) {
-        const unsigned k = k0 + it * p.nt;
+    for (unsigned k = k0; k < k1; k += step) {
         const Vel v = load_vel<D>(p, k, vt);
         const double s = dotnc(v.x, v.y, v.z, S);
         if (s > 0) continue;
+        double gin, hin;
         if (sym) {
             const unsigned km = p.mir[(size_t)fx.N * p.nvp + k];
             const Vel vm = load_vel<D>(p, km, vt);
@@ -964,15 +997,32 @@ __global__ __launch_bounds__(MAXNT) void k_face_open(P<TS> p)
             const double hm = H ? ld(hrowC, km) : 0.0;
             double GM[3] = {0, 0, 0}, HM[3] = {0, 0, 0};
             grad_at<D, H, NS>(p, c, km, gm, hm, GM, HM);
-            st_stream(fg, k, gm + dotg<D>(GM, dP, hxm));
-            if (H) st_stream(fh, k, hm + dotg<D>(HM, dP, hxm));
+            gin = gm + dotg<D>(GM, dP, hxm);
+            hin = H ? hm + dotg<D>(HM, dP, hxm) : 0.0;
         } else {
             const double cx = Ui[0] - v.x, cy = Ui[1] - v.y, cz = Ui[2] - v.z;
-            const double gin = W.rho_b * (W.pre * exp(-(cx * cx + cy * cy + cz * cz) / (2.0 * RT)));
-            st_stream(fg, k, gin - row_off<D>(p, v, 0, vt));
-            if (H) st_stream(fh, k, gin * RT * p.kc - row_off<D>(p, v, 1, vt));
+            const double m = W.rho_b * (W.pre * exp(-(cx * cx + cy * cy + cz * cz) / (2.0 * RT)));
+            gin = m - row_off<D>(p, v, 0, vt);
+            hin = H ? m * RT * p.kc - row_off<D>(p, v, 1, vt) : 0.0;
         }
+        st_stream(fg, k, gin);
+        if (H) st_stream(fh, k, hin);
+        if (MOM)
+            acc_moments<D, H>(acc, (double)(TS)gin + row_off<D>(p, v, 0, vt),
+                              H ? (double)(TS)hin + row_off<D>(p, v, 1, vt) : 0.0, v, Uo);
     }
+}
+
+template <int D, bool H, int NS, typename TS>
+__global__ __launch_bounds__(MAXNT) void k_face_open(P<TS> p)
+{
+    __shared__ double vt[VT_SIZE];
+    const int i = blockIdx.x, b = blockIdx.y;
+    if (i >= p.nopen || b >= p.nb) return;
+    stage_vt(p, vt);
+    __syncthreads();
+    const unsigned k0 = (unsigned)b * p.vb;
+    open_face<D, H, NS, false>(p, i, k0 + threadIdx.x, k0 + (unsigned)p.nib * p.nt, p.nt, vt, nullptr);
 }
 
 // k_face_moments: face-wise, over one velocity block: the S6 moment sums and the wall outGoing
@@ -1183,17 +1233,26 @@ __global__ __launch_bounds__(MX_NT) void k_face_moments_mx(P<TS> p)
     }
 }
 
+#include "lines.h"
+
 // ---------------------------------------------------------------------------------------------
 // k_face_fin: one thread per face.  Sums the block partials in block order, then S3 wall density
 // rho_w = outGoing / |inComingByRho| (calculatedMaxwellFvPatchField.C:139-164) with the moments of
 // the S4 incoming Maxwellian added, the S6 face macros (fvDVM.C:456-522), the S7 equilibrium
 // constants and relaxation factor, and the wall diagnostics qWall, stressWall (fvDVM.C:539-581).
+// LINES: the sums are the moment records of the face's cells (each about its cell's velocity) and
+// of its open incoming half, shifted to the face's reference velocity; outGoing = S . momentum of a
+// wall's outgoing values.
 // ---------------------------------------------------------------------------------------------
-template <int D, typename TS>
+template <int D, typename TS, bool LINES = false>
 __global__ __launch_bounds__(256) void k_face_fin(P<TS> p)
 {
     constexpr int NM = NMom<D>::v + 1;
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
+    if (LINES && f >= p.nf) {
+        if (f - p.nf < p.nc) line_cell<D>(p, f - p.nf);
+        return;
+    }
     if (f >= p.nf) return;
     const FaceX &fx = p.fx[f];
     const bool wall = fx.kind == KIND_WALL;
@@ -1201,18 +1260,30 @@ __global__ __launch_bounds__(256) void k_face_fin(P<TS> p)
     const double dt = p.dtc[cas];
     double a[NM];
     for (int m = 0; m < NM; ++m) a[m] = 0.0;
-    const double *fp = p.fpart + (size_t)f * p.nb * NM;
-    for (int b = 0; b < p.nb; ++b)
-        for (int m = 0; m < NM; ++m) a[m] += fp[b * NM + m];
     double Uh[3];
     double rho_w = 0.0;
     if (wall) {
         const WallC &W = p.wall[fx.bidx];
         Uh[0] = W.U[0]; Uh[1] = W.U[1]; Uh[2] = W.U[2];
-        rho_w = a[NM - 1] / fabs(W.incoming);
-        for (int m = 0; m < NM - 1; ++m) a[m] = fma(rho_w, W.A[m], a[m]);
     } else {
         Uh[0] = p.fU[3 * f]; Uh[1] = p.fU[3 * f + 1]; Uh[2] = p.fU[3 * f + 2];
+    }
+    if (LINES) {
+        const int4 q = p.fslot[f];
+        record_add<D>(a, p.spart + (size_t)q.x * (NM - 1), p.cU + 3 * (size_t)fx.P, Uh);
+        if (q.y >= 0) record_add<D>(a, p.spart + (size_t)q.y * (NM - 1), p.cU + 3 * (size_t)fx.N, Uh);
+        if (q.z >= 0) record_add<D>(a, p.opart + (size_t)q.z * (NM - 1), p.cU + 3 * (size_t)fx.P, Uh);
+        if (wall)
+            for (int d = 0; d < D; ++d) a[NM - 1] += fx.S[d] * a[1 + d];
+    } else {
+        const double *fp = p.fpart + (size_t)f * p.nb * NM;
+        for (int b = 0; b < p.nb; ++b)
+            for (int m = 0; m < NM; ++m) a[m] += fp[b * NM + m];
+    }
+    if (wall) {
+        const WallC &W = p.wall[fx.bidx];
+        rho_w = a[NM - 1] / fabs(W.incoming);
+        for (int m = 0; m < NM - 1; ++m) a[m] = fma(rho_w, W.A[m], a[m]);
     }
     double rho, U[3], T, tau, q[3];
     finish_moments<D>(a, Uh, p.R, p.K, p.muc[cas], p.omega, p.Tref, rho, U, T, tau, q);
@@ -1273,6 +1344,21 @@ __global__ __launch_bounds__(256) void k_face_fin(P<TS> p)
             }
     }
     p.feq[f] = fe;
+    if (LINES) {
+        const int4 q = p.fslot[f];
+        LineFace lf;
+        lf.invRT = fe.invRT;
+        lf.B = fe.B[D - 1];
+        lf.qz = fe.qc[D - 1];
+        lf.omr = fe.omr;
+        lf.RT = fe.RT;
+        lf.pad[0] = lf.pad[1] = 0.0;
+        for (int side = 0; side < (q.y >= 0 ? 2 : 1); ++side) {
+            const double f = side ? dt / p.cV[fx.N] : -(dt / p.cV[fx.P]);
+            lf.Sl = fx.S[D - 1] * f;
+            p.lface[side ? q.y : q.x] = lf;
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1847,6 +1933,19 @@ struct dugks_engine {
     int nmx_tiles = 0, nwallf = 0;
     int face_mfma = 1;   // FP64 face-value mode: face moments on the matrix cores
     double *fpart = nullptr, *cpart = nullptr;
+    // velocity columns (lines.h)
+    int line_ok = 0;     // the mesh and the velocity set fit the column kernels
+    int ntile = 0, line_w = 1;   // tiles; waves per cell
+    LineRec *rec = nullptr;
+    int *titer = nullptr;
+    std::vector<int> titer_h;
+    int nvp_img = 0;     // padded velocity count of a state image's rows
+    int *img_slot = nullptr;
+    LineGeo *lgeo = nullptr;
+    double *spart = nullptr, *opart = nullptr;
+    LineFace *lface = nullptr;
+    LineCell *lcell = nullptr;
+    int4 *fslot = nullptr;
     void *gb[2] = {nullptr, nullptr}, *hb[2] = {nullptr, nullptr};
     void *gB[2] = {nullptr, nullptr}, *hB[2] = {nullptr, nullptr};
     int face_values = 0;  // face-value mode: the face values are stored, k_cell reads them
@@ -1949,6 +2048,8 @@ P<TS> params(dugks_engine *h)
     p.fsel = nullptr;
     p.nfsel = 0;
     p.mxf = h->mxf;
+    p.rec = h->rec; p.titer = h->titer; p.lgeo = h->lgeo; p.ntile = h->ntile; p.ntl = 0;
+    p.spart = h->spart; p.opart = h->opart; p.lface = h->lface; p.lcell = h->lcell; p.fslot = h->fslot;
     p.fvg = h->face_values ? (TS *)h->fvg : nullptr;
     p.fvh = h->face_values ? (TS *)h->fvh : nullptr;
     p.flag = h->flag;
@@ -2028,9 +2129,86 @@ void launch_step_fv(dugks_engine *h, hipEvent_t *ev)
     if (ev) (void)hipEventRecord(ev[6], h->stream);
 }
 
+// Column kernels run in face-value mode with the default face moments.
+bool use_lines(const dugks_engine *h) { return h->line_ok && h->face_values && h->face_mfma && !h->face_pass_legacy; }
+
+// LDS bytes of the column kernels (k_cell_lines: without the new row)
+template <int D, bool H, int NS>
+size_t line_face_lds(const dugks_engine *h, int waves)
+{
+    const size_t sums = 6 * (size_t)h->nxi + (size_t)waves * NS * line_nval<D, H>();
+    return 8 * (3 * (size_t)h->nax + 2 + std::max(sums, (size_t)(waves + 1) * NMom<D>::v));
+}
+
+template <int D, int NS>
+size_t line_cell_lds(const dugks_engine *h)
+{
+    const size_t la0 = (size_t)(D - 1) * h->nxi;
+    return 8 * (3 * (size_t)h->nax + 2 + line_lt<NS>() * (size_t)h->nxi + (NS + 1) * la0 + NS * (size_t)h->nax);
+}
+
+template <int D, bool H, int NS, typename TS>
+void launch_step_lines(dugks_engine *h, hipEvent_t *ev)
+{
+    P<TS> p = params<TS>(h);
+    p.nb = p.nbc = 1;
+    p.vb = h->nvp;
+    p.nib = h->nvp / h->nt;
+    const int w = h->line_w;
+    if (ev) (void)hipEventRecord(ev[0], h->stream);
+    // the open faces' blocks first, as many as keep the cells' blocks on their XCDs
+    dim3 grid = block_grid(h->nc, 1);
+    grid.x += block_grid(h->nopen, 1).x;
+    hipLaunchKernelGGL((k_face_lines<D, H, NS, TS>), grid, dim3(64 * w), (line_face_lds<D, H, NS>(h, w)), h->stream, p);
+    if (ev) (void)hipEventRecord(ev[1], h->stream);
+    if (ev) (void)hipEventRecord(ev[2], h->stream);
+    // a thread per face or cell and little work each: small workgroups spread it over more CUs
+    hipLaunchKernelGGL((k_face_fin<D, TS, true>), dim3((h->nf + h->nc + 63) / 64), dim3(64), 0, h->stream, p);
+    if (ev) (void)hipEventRecord(ev[3], h->stream);
+    // The new row of the first ntl tiles stays in LDS until S1: as many as fit without costing a
+    // workgroup (16 waves a CU, 12 where the kernel takes 168 registers; fewer resident waves cost more than the saved row traffic:
+    // 64 cavities of 28^2 velocities 3.1 -> 4.1 ms with the whole row in LDS).
+    size_t lds = line_cell_lds<D, NS>(h);
+    const size_t es = sizeof(TS) * (H ? 2 : 1);
+    const int wgs = std::max(1, (D == 3 && H ? 12 : 16) / w);
+    const size_t cap = LDS_CU / wgs - 2048;
+    while (h->fuse_s1 && p.ntl < h->ntile && lds + h->titer_h[p.ntl + 1] * 64 * es <= cap) ++p.ntl;
+    lds += h->titer_h[p.ntl] * 64 * es;
+    auto launch_cell = [&](auto f1) {
+        hipLaunchKernelGGL((k_cell_lines<D, H, NS, TS, decltype(f1)::value>), block_grid(h->nc, 1), dim3(64 * w), lds,
+                           h->stream, p);
+    };
+    if (h->fuse_s1) {
+        launch_cell(std::true_type{});
+        if (ev) (void)hipEventRecord(ev[4], h->stream);
+        if (h->npress)
+            hipLaunchKernelGGL((k_pressure_bc<D, TS>), dim3((h->nopen + 255) / 256), dim3(256), 0, h->stream, p);
+        if (ev) (void)hipEventRecord(ev[5], h->stream);
+        if (ev) (void)hipEventRecord(ev[6], h->stream);
+        return;
+    }
+    launch_cell(std::false_type{});
+    if (ev) (void)hipEventRecord(ev[4], h->stream);
+    hipLaunchKernelGGL((k_cell_fin<D, TS>), dim3((h->nc + 255) / 256), dim3(256), 0, h->stream, p);
+    if (h->npress)
+        hipLaunchKernelGGL((k_pressure_bc<D, TS>), dim3((h->nopen + 255) / 256), dim3(256), 0, h->stream, p);
+    if (ev) (void)hipEventRecord(ev[5], h->stream);
+    hipLaunchKernelGGL((k_cell_s1_lines<D, H, TS>), dim3(h->nc), dim3(64 * w), 0, h->stream, p);
+    if (ev) (void)hipEventRecord(ev[6], h->stream);
+}
+
 template <int D, bool H, int NS, typename TS>
 void launch_step_ns(dugks_engine *h, hipEvent_t *ev)
 {
+    if constexpr (NS <= 6) {
+        if (use_lines(h)) {
+            if constexpr (D == 1) return launch_step_lines<D, H, 2, TS>(h, ev);
+            else if constexpr (D == 2) {
+                if (h->ns_max <= 3) return launch_step_lines<D, H, 3, TS>(h, ev);
+                return launch_step_lines<D, H, 4, TS>(h, ev);
+            } else return launch_step_lines<D, H, NS, TS>(h, ev);
+        }
+    }
     if (h->face_values) launch_step_fv<D, H, NS, TS, true>(h, ev);
     else launch_step_fv<D, H, NS, TS, false>(h, ev);
 }
@@ -2247,6 +2425,117 @@ void shape_candidates(dugks_engine *h)
     h->nbc_cap = h->nvbc;
     for (auto &c : h->face_cand) h->nb_cap = std::max(h->nb_cap, h->nvp / (c.first * c.second));
     h->nbc_cap = h->nb_cap = std::max(h->nb_cap, h->nbc_cap);
+}
+
+// Velocity columns of the tensor set (lines.h): the lanes of every tile, the iterations before each
+// tile, and the velocity (reference index, -1 padding) of every slot of a row.  A column has fixed
+// (x, y) (3-D) or x (2-D) and runs over every m-th velocity of the last axis.  Columns are ordered by
+// the sign classes of their fixed axes, so that the upwind side of an axis-aligned face is uniform over
+// runs of lanes.
+//
+// m and the waves per cell (w) are those of the least cost, in iterations of a wave:
+//   - a tile costs its iterations and TILE_COST (set-up, final lane sums; 12^3 velocities FP32, 26^3 cells:
+//     917 us with 3 tiles of 27 iterations in all, 1130 with 14), and in 2-D MIX_COST more an iteration
+//     where a change of sign class lies inside a 128-byte line, which two cells then write in part (28^2
+//     velocities, 64 cavities: 5.09 ms with 10 such iterations of 13, 4.80 with 6 of 13);
+//   - a wave costs its tiles and WAVE_COST, and more where it is long: a tenth each time its length doubles
+//     past 13 (16^3 velocities, 30^3 cells: 2.97 ms with 1 wave of 64 iterations, 2.74 with 2; 24^3, 24^3:
+//     5.30 with 1 wave of 216, 4.44 with 3), a third where all waves run at once, each phase
+//     together (60^2 cells of 41^2: 304 us with 1, 247 with 2);
+//   - all cells cost that times the rounds of waves the device needs (48^2 cells of 35^2 velocities: 150,
+//     160 and 140 us with 1, 2 and 3 waves a cell, 1, 2 and 2 rounds); past a few rounds the last one's
+//     idle half is what counts.
+// At most 4 waves a cell: 48^3 cells of 24^3 velocities take 34.4 ms with 3, 49.7 with 5.
+constexpr double TILE_COST = 0.8, MIX_COST = 0.2, WAVE_COST = 2.0;
+
+void velocity_columns(int D, int nxi, const double *xi, int nc, int slots, int line, std::vector<LineRec> &recs,
+                      std::vector<int> &titer, std::vector<int> &slot_ref, int &waves)
+{
+    auto sgn = [](double x) { return x < 0 ? 0 : (x == 0 ? 1 : 2); };
+    std::vector<int> ax[3];   // axis indices by sign class
+    for (int i = 0; i < nxi; ++i) ax[sgn(xi[i])].push_back(i);
+    struct Col { int ix, iy, l, dl, n; };
+    // every m-th velocity of the columns i0, i0 + 1, ... of v
+    auto split = [](const std::vector<Col> &v, size_t i0, int m) {
+        std::vector<Col> r;
+        for (int s = 0; s < m; ++s)
+            for (size_t i = i0; i < v.size(); ++i)
+                if (v[i].n > s) r.push_back({v[i].ix, v[i].iy, v[i].l + s * v[i].dl, v[i].dl * m, (v[i].n - s + m - 1) / m});
+        return r;
+    };
+    std::vector<Col> best;
+    double best_cost = -1.0;
+    for (int m = 1; m <= nxi; ++m) {
+        // 2-D: at least 24 lanes of one sign class together where there are as many: 14-lane runs (28 points,
+        // m = 1) take the batch's face pass 3.1 ms, 28-lane runs 2.3 ms (partly written cache lines)
+        if (D == 2 && m * (int)ax[2].size() < 24 && m < nxi) continue;
+        std::vector<Col> v;
+        for (int cy = 0; cy < (D == 3 ? 3 : 1); ++cy)
+            for (int cx = 0; cx < (D >= 2 ? 3 : 1); ++cx) {
+                std::vector<Col> q;
+                for (int y = 0; y < (D == 3 ? (int)ax[cy].size() : 1); ++y)
+                    for (int x = 0; x < (D >= 2 ? (int)ax[cx].size() : 1); ++x)
+                        q.push_back({D >= 2 ? ax[cx][x] : 0, D == 3 ? ax[cy][y] : 0, 0, 1, nxi});
+                q = split(q, 0, m);
+                v.insert(v.end(), q.begin(), q.end());
+            }
+        // the columns of a last partial tile are split further, over its idle lanes
+        const size_t full = v.size() / 64 * 64, left = v.size() - full;
+        if (left) {
+            const std::vector<Col> q = split(v, full, std::min((int)(64 / left), v[full].n));
+            v.resize(full);
+            v.insert(v.end(), q.begin(), q.end());
+        }
+        std::vector<double> tile;
+        for (size_t i = 0; i < v.size(); i += 64) {
+            const size_t i1 = std::min(v.size(), i + 64);
+            int its = 0;
+            bool mix = false;
+            for (size_t k = i; k < i1; ++k) {
+                its = std::max(its, v[k].n);
+                mix = mix || (D == 2 && k % line && sgn(xi[v[k].ix]) != sgn(xi[v[k - 1].ix]));
+            }
+            tile.push_back(its * (mix ? 1 + MIX_COST : 1) + TILE_COST);
+        }
+        for (int w = 1; w <= std::min(4, (int)tile.size()); ++w) {
+            std::vector<double> busy(w, WAVE_COST);
+            for (size_t t = 0; t < tile.size(); ++t) busy[t % w] += tile[t];
+            const double b = *std::max_element(busy.begin(), busy.end());
+            const double x = (double)nc * w / slots, rounds = x < 3 ? std::ceil(x) : x + 0.5;
+            const double lone = 0.35 * std::min(1.0, std::max(0.0, (b - 20) / 13)), tail = 0.1 * std::max(0.0, std::log2(b / 13));
+            const double cost = rounds * b * (1 + (x <= 1 ? lone : tail));
+            if (best_cost < 0 || cost < best_cost) {
+                best = v;
+                best_cost = cost;
+                waves = w;
+            }
+        }
+    }
+    titer.assign(1, 0);
+    for (size_t i0 = 0; i0 < best.size(); i0 += 64) {
+        const int q0 = titer.back();
+        int its = 0;
+        for (size_t i = i0; i < std::min(best.size(), i0 + 64); ++i) its = std::max(its, best[i].n);
+        slot_ref.resize((size_t)(q0 + its) * 64, -1);
+        for (size_t i = i0; i < i0 + 64; ++i) {
+            LineRec r{0, 0, 0, 0, 0};
+            if (i < best.size()) {
+                const Col &q = best[i];
+                r.ix = (uint8_t)q.ix;
+                r.iy = (uint8_t)q.iy;
+                r.l = (uint8_t)q.l;
+                r.dl = (uint8_t)q.dl;
+                r.n = q.n;
+                for (int k = 0; k < q.n; ++k) {
+                    const int l = q.l + k * q.dl;
+                    slot_ref[(size_t)(q0 + k) * 64 + (i - i0)] =
+                        D == 3 ? (l * nxi + q.iy) * nxi + q.ix : (D == 2 ? l * nxi + q.ix : l);
+                }
+            }
+            recs.push_back(r);
+        }
+        titer.push_back(q0 + its);
+    }
 }
 
 using dugks_lsq::mag3;
@@ -2530,7 +2819,37 @@ int build(dugks_engine *h, const dugks_case *cs)
         int kb = cls(rz[b]) * 9 + cls(ry[b]) * 3 + cls(rx[b]);
         return ka < kb;
     });
+    // ---- row layout ----
+    // Sign-sorted velocities, or (meshes and options of the column kernels) the slots of their tiles,
+    // where the face values fit as they have to for face-value mode to be the default.
     choose_blocks(nv, h->nt, h->nib, h->nvb, h->nvp);
+    h->nvp_img = h->nvp;
+    h->ns_max = 0;
+    for (int c = 0; c < nc; ++c) h->ns_max = std::max(h->ns_max, cnt[c + 1] - cnt[c]);
+    std::vector<LineRec> recs;
+    std::vector<int> slot_ref(order);
+    h->titer_h.assign(1, 0);
+    {
+        const char *fm = std::getenv("DUGKS_FACE_MFMA"), *fl = std::getenv("DUGKS_FACE_PASS_LEGACY"),
+                   *fv = std::getenv("DUGKS_FACE_VALUES");
+        std::vector<int> refs;
+        size_t fr = 0, tot = 0;
+        h->line_ok = h->ns_max <= (D == 3 ? 6 : (D == 2 ? 4 : 2)) && !(fm && !std::atoi(fm)) && !(fl && std::atoi(fl)) &&
+                     !(fv && !std::atoi(fv)) && hipSetDevice(cs->device) == hipSuccess && hipMemGetInfo(&fr, &tot) == hipSuccess;
+        if (h->line_ok) {
+            velocity_columns(D, nxi, cs->xi, nc, NCU * (D == 3 && h->has_h ? 12 : 16), 128 / (int)ts_size(h), recs,
+                             h->titer_h, refs, h->line_w);
+            // the resident rows take their part of the free memory first
+            const double es = (double)ts_size(h) * (h->has_h ? 2 : 1) * refs.size();
+            h->line_ok = es * nf <= 0.5 * ((double)fr - 2.0 * es * ((double)nc + h->nw) - 2048.0 * ((double)nc + nf));
+        }
+        if (h->line_ok) {
+            h->ntile = (int)h->titer_h.size() - 1;
+            slot_ref = refs;
+            choose_blocks((int)refs.size(), h->nt, h->nib, h->nvb, h->nvp);
+        }
+    }
+    slot_ref.resize(h->nvp, -1);
     h->vb = h->nt * h->nib;
     h->niter = h->nvb * h->nib;
     shape_candidates(h);
@@ -2541,16 +2860,15 @@ int build(dugks_engine *h, const dugks_case *cs)
         return fail(h, DUGKS_ERR_UNSUPPORTED, "mesh too large for one dispatch per kernel");
     // ---- least-squares stencils (entry j = slot j; rows: cells, then walls) ----
     std::vector<CellSt> cst(nc);
-    h->ns_max = 0;
     for (int c = 0; c < nc; ++c) {
         CellSt t;
         std::memset(&t, 0, sizeof t);
         const int ns = cnt[c + 1] - cnt[c];
-        h->ns_max = std::max(h->ns_max, ns);
-        t.inner = ns > 0;
+        t.inner = t.plain = ns > 0;
         for (int j = 0; j < ns; ++j) {
             const int kd = sl[cnt[c] + j].kind;
             if (kd != KIND_OWN && kd != KIND_NEI) t.inner = 0;
+            if (kd != KIND_OWN && kd != KIND_NEI && kd != KIND_CYC) t.plain = 0;
         }
         for (int j = 0; j < MAXS; ++j) {
             t.off[j] = (int64_t)c * h->nvp;
@@ -2573,21 +2891,48 @@ int build(dugks_engine *h, const dugks_case *cs)
     }
     const int nvp = h->nvp;
     std::vector<uint32_t> vidx(nvp, VPAD);
-    h->perm.assign(nvp, -1);
-    for (int k = 0; k < nv; ++k) {
-        const int r = order[k];
-        vidx[k] = (uint32_t)rid[r];
-        h->perm[k] = r;
+    h->perm = slot_ref;
+    std::vector<int> img_slot(h->nvp_img, -1);   // state image: sign-sorted velocity -> slot
+    {
+        std::vector<int> slot(nv);
+        for (int k = 0; k < nvp; ++k)
+            if (slot_ref[k] >= 0) {
+                vidx[k] = (uint32_t)rid[slot_ref[k]];
+                slot[slot_ref[k]] = k;
+            }
+        for (int k = 0; k < nv; ++k) img_slot[k] = slot[order[k]];
     }
+    const int lns = D == 1 ? 2 : (D == 2 ? (h->ns_max <= 3 ? 3 : 4) : 6);   // slots per cell of the column kernels
+    std::vector<int4> fslot(nf, int4{-1, -1, -1, 0});
+    std::vector<LineGeo> lgeo(h->line_ok ? (size_t)nc * lns : 0);
+    for (int c = 0; c < nc && h->line_ok; ++c)
+        for (int j = 0; j < lns; ++j) {
+            LineGeo &g = lgeo[(size_t)c * lns + j];
+            std::memset(&g, 0, sizeof g);
+            g.face = sl[cnt[c]].face;
+            g.kind = KIND_OWN;
+            if (cnt[c] + j >= cnt[c + 1]) continue;
+            const Slot &q = sl[cnt[c] + j];
+            const double sgn = q.kind == KIND_NEI ? -1.0 : 1.0;
+            g.face = q.face;
+            g.kind = q.kind;
+            for (int d = 0; d < 3; ++d) g.dC[d] = q.dCs[d];
+            for (int d = 0; d + 1 < D; ++d) g.S[d] = sgn * q.S[d];
+            g.Sl = sgn * q.S[D - 1];
+            (q.kind == KIND_NEI ? fslot[q.face].y : fslot[q.face].x) = c * lns + j;
+        }
+    for (size_t i = 0; i < open_faces.size(); ++i) fslot[open_faces[i]].z = (int)i;
     // mirrored velocities (symmXtgID / symmYtgID / symmZtgID, fvDVM.C:152-166, 183-195) in device order
     std::vector<uint32_t> mir(3 * (size_t)nvp);
     {
         std::vector<int> inv(nv);
-        for (int k = 0; k < nv; ++k) inv[h->perm[k]] = k;
+        for (int k = 0; k < nvp; ++k)
+            if (h->perm[k] >= 0) inv[h->perm[k]] = k;
         for (int k = 0; k < nvp; ++k)
             for (int a = 0; a < 3; ++a) mir[(size_t)a * nvp + k] = (uint32_t)k;
-        for (int k = 0; k < nv; ++k) {
+        for (int k = 0; k < nvp; ++k) {
             const int r = h->perm[k];
+            if (r < 0) continue;
             const int ix = r % nxi, iy = D >= 2 ? (r / nxi) % nxi : 0, iz = D == 3 ? r / (nxi * nxi) : 0;
             const int ny = D >= 2 ? nxi : 1, nz = D == 3 ? nxi : 1;
             mir[k] = (uint32_t)inv[(iz * ny + iy) * nxi + (nxi - 1 - ix)];
@@ -2694,6 +3039,21 @@ int build(dugks_engine *h, const dugks_case *cs)
         (r = upload(h, h->fx, fxs.data(), nf)) || (r = upload(h, h->cst, cst.data(), nc)) ||
         (r = upload(h, h->corder, corder.data(), nc)) || (r = upload(h, h->forder, forder.data(), nf)) || (r = upload(h, h->wfslot, wfslot.data(), nw)))
         return r;
+    // rows are padded to nvp; the column kernels write the nv velocities only, the others read the
+    // padding with weight 0
+    for (int i = 0; i < 2; ++i) {
+        HIPCHK(h, hipMemset(h->gb[i], 0, row + brow));
+        if (h->has_h) HIPCHK(h, hipMemset(h->hb[i], 0, row + brow));
+    }
+    if (h->line_ok &&
+        ((r = dalloc(h, &h->img_slot, img_slot.size())) || (r = upload(h, h->img_slot, img_slot.data(), img_slot.size())) ||
+         (r = dalloc(h, &h->rec, recs.size())) || (r = upload(h, h->rec, recs.data(), recs.size())) ||
+         (r = dalloc(h, &h->titer, h->titer_h.size())) || (r = upload(h, h->titer, h->titer_h.data(), h->titer_h.size())) ||
+         (r = dalloc(h, &h->lgeo, lgeo.size())) || (r = upload(h, h->lgeo, lgeo.data(), lgeo.size())) ||
+         (r = dalloc(h, &h->spart, (size_t)nc * lns * NMom<3>::v)) ||
+         (r = dalloc(h, &h->opart, open_faces.size() * NMom<3>::v)) || (r = dalloc(h, &h->lface, (size_t)nc * lns)) || (r = dalloc(h, &h->lcell, (size_t)nc)) ||
+         (r = dalloc(h, &h->fslot, nf)) || (r = upload(h, h->fslot, fslot.data(), nf))))
+        return r;
     if (nw && (r = upload(h, h->wall, wc.data(), nw))) return r;
     if (nw && ((r = dalloc(h, &h->bpress, nw)) || (r = upload(h, h->bpress, wpress.data(), nw)))) return r;
     h->nopen = (int)open_faces.size();
@@ -2746,6 +3106,7 @@ void release(dugks_engine *h)
     dfree(h->ctau); dfree(h->frho); dfree(h->fU); dfree(h->fT); dfree(h->fq); dfree(h->feq);
     dfree(h->wall); dfree(h->wexp); dfree(h->qwall); dfree(h->swall); dfree(h->fx); dfree(h->cst);
     dfree(h->corder); dfree(h->forder); dfree(h->fpart); dfree(h->cpart); dfree(h->mxf); dfree(h->wallf);
+    dfree(h->rec); dfree(h->titer); dfree(h->img_slot); dfree(h->lgeo); dfree(h->spart); dfree(h->opart); dfree(h->lface); dfree(h->lcell); dfree(h->fslot);
     for (int i = 0; i < 2; ++i) {
         dfree(h->gb[i]); dfree(h->hb[i]);
         h->gB[i] = h->hB[i] = nullptr;
@@ -2921,6 +3282,28 @@ int step_impl(dugks_engine *h, const double *dtc, int nsteps)
         h->prof_steps += nsteps;
     }
     return r;
+}
+
+// Rows of the current state <-> rows of a state image (sign-sorted velocities, nvp_img a row), for the
+// column layout.  The other ping-pong side, which holds nothing between steps, stages them.
+template <typename TS>
+__global__ __launch_bounds__(256) void k_image(TS *img, TS *rows, const int *slot, int nimg, int nvp, int save)
+{
+    TS *a = img + (size_t)blockIdx.x * nimg, *r = rows + (size_t)blockIdx.x * nvp;
+    for (int k = threadIdx.x; k < nimg; k += blockDim.x) {
+        const int q = slot[k];
+        if (save) a[k] = q >= 0 ? r[q] : (TS)0;
+        else if (q >= 0) r[q] = a[k];
+    }
+}
+
+void image_rows(dugks_engine *h, void *img, void *rows, int save)
+{
+    const int n = h->nc + (h->nw ? h->nw : 1);
+    if (h->storage == DUGKS_STORAGE_FP32)
+        hipLaunchKernelGGL((k_image<float>), dim3(n), dim3(256), 0, h->stream, (float *)img, (float *)rows, h->img_slot, h->nvp_img, h->nvp, save);
+    else
+        hipLaunchKernelGGL((k_image<double>), dim3(n), dim3(256), 0, h->stream, (double *)img, (double *)rows, h->img_slot, h->nvp_img, h->nvp, save);
 }
 
 const int64_t STATE_MAGIC = 0x44554b5331LL;  // "DUKS1"
@@ -3264,8 +3647,8 @@ int dugks_state_size(dugks_engine *h, int64_t *bytes)
     const int64_t es = (int64_t)ts_size(h);
     const int64_t nh = h->has_h ? 2 : 1;
     int64_t n = 16 * 8;
-    n += nh * (int64_t)h->nc * h->nvp * es;
-    n += nh * (int64_t)(h->nw ? h->nw : 1) * h->nvp * es;
+    n += nh * (int64_t)h->nc * h->nvp_img * es;
+    n += nh * (int64_t)(h->nw ? h->nw : 1) * h->nvp_img * es;
     n += 9 * (int64_t)h->nc * 8 + 3 * (int64_t)h->nf * 8 + (int64_t)h->n_cases * 8;
     n += (int64_t)h->nw * (int64_t)sizeof(WallC);   // pressure patches evolve their boundary state
     *bytes = n;
@@ -3281,17 +3664,25 @@ int dugks_save_state(dugks_engine *h, void *buf, int64_t bytes)
     HIPCHK(h, hipSetDevice(h->device));
     HIPCHK(h, hipStreamSynchronize(h->stream));
     char *p = (char *)buf;
-    int64_t hdr[16] = {STATE_MAGIC, h->nc, h->nvp, h->nw, h->nf, h->storage, h->has_h, h->raw, h->n_cases, h->D, 0, 0, 0, 0, 0, 0};
+    int64_t hdr[16] = {STATE_MAGIC, h->nc, h->nvp_img, h->nw, h->nf, h->storage, h->has_h, h->raw, h->n_cases, h->D, 0, 0, 0, 0, 0, 0};
     std::memcpy(&hdr[10], &h->off_rho, sizeof(double));   // FP32 row offsets travel with the rows
     std::memcpy(&hdr[11], &h->off_T, sizeof(double));
     std::memcpy(p, hdr, sizeof hdr);
     p += sizeof hdr;
     const size_t es = ts_size(h);
-    const size_t row = (size_t)h->nc * h->nvp * es, brow = (size_t)(h->nw ? h->nw : 1) * h->nvp * es;
-    HIPCHK(h, hipMemcpy(p, h->gb[h->cur], row, hipMemcpyDeviceToHost)); p += row;
-    if (h->has_h) { HIPCHK(h, hipMemcpy(p, h->hb[h->cur], row, hipMemcpyDeviceToHost)); p += row; }
-    HIPCHK(h, hipMemcpy(p, h->gB[h->cur], brow, hipMemcpyDeviceToHost)); p += brow;
-    if (h->has_h) { HIPCHK(h, hipMemcpy(p, h->hB[h->cur], brow, hipMemcpyDeviceToHost)); p += brow; }
+    const size_t row = (size_t)h->nc * h->nvp_img * es, brow = (size_t)(h->nw ? h->nw : 1) * h->nvp_img * es;
+    const int side = h->line_ok ? 1 - h->cur : h->cur;
+    if (h->line_ok) {
+        image_rows(h, h->gb[side], h->gb[h->cur], 1);
+        if (h->has_h) image_rows(h, h->hb[side], h->hb[h->cur], 1);
+        HIPCHK(h, hipGetLastError());
+        HIPCHK(h, hipStreamSynchronize(h->stream));
+    }
+    const char *gr = (const char *)h->gb[side], *hr = (const char *)h->hb[side];   // cell rows, then wall rows
+    HIPCHK(h, hipMemcpy(p, gr, row, hipMemcpyDeviceToHost)); p += row;
+    if (h->has_h) { HIPCHK(h, hipMemcpy(p, hr, row, hipMemcpyDeviceToHost)); p += row; }
+    HIPCHK(h, hipMemcpy(p, gr + row, brow, hipMemcpyDeviceToHost)); p += brow;
+    if (h->has_h) { HIPCHK(h, hipMemcpy(p, hr + row, brow, hipMemcpyDeviceToHost)); p += brow; }
     const size_t nc = h->nc;
     HIPCHK(h, hipMemcpy(p, h->crho, 8 * nc, hipMemcpyDeviceToHost)); p += 8 * nc;
     HIPCHK(h, hipMemcpy(p, h->cU, 24 * nc, hipMemcpyDeviceToHost)); p += 24 * nc;
@@ -3315,18 +3706,26 @@ int dugks_load_state(dugks_engine *h, const void *buf, int64_t bytes)
     const char *p = (const char *)buf;
     int64_t hdr[16];
     std::memcpy(hdr, p, sizeof hdr);
-    if (hdr[0] != STATE_MAGIC || hdr[1] != h->nc || hdr[2] != h->nvp || hdr[3] != h->nw || hdr[4] != h->nf ||
+    if (hdr[0] != STATE_MAGIC || hdr[1] != h->nc || hdr[2] != h->nvp_img || hdr[3] != h->nw || hdr[4] != h->nf ||
         hdr[5] != h->storage || hdr[6] != (int64_t)h->has_h || hdr[8] != h->n_cases || hdr[9] != h->D)
         return fail(h, DUGKS_ERR_INVALID, "state image does not match this engine");
     p += sizeof hdr;
     HIPCHK(h, hipSetDevice(h->device));
     HIPCHK(h, hipStreamSynchronize(h->stream));
     const size_t es = ts_size(h);
-    const size_t row = (size_t)h->nc * h->nvp * es, brow = (size_t)(h->nw ? h->nw : 1) * h->nvp * es;
-    HIPCHK(h, hipMemcpy(h->gb[h->cur], p, row, hipMemcpyHostToDevice)); p += row;
-    if (h->has_h) { HIPCHK(h, hipMemcpy(h->hb[h->cur], p, row, hipMemcpyHostToDevice)); p += row; }
-    HIPCHK(h, hipMemcpy(h->gB[h->cur], p, brow, hipMemcpyHostToDevice)); p += brow;
-    if (h->has_h) { HIPCHK(h, hipMemcpy(h->hB[h->cur], p, brow, hipMemcpyHostToDevice)); p += brow; }
+    const size_t row = (size_t)h->nc * h->nvp_img * es, brow = (size_t)(h->nw ? h->nw : 1) * h->nvp_img * es;
+    const int side = h->line_ok ? 1 - h->cur : h->cur;
+    char *gr = (char *)h->gb[side], *hr = (char *)h->hb[side];
+    HIPCHK(h, hipMemcpy(gr, p, row, hipMemcpyHostToDevice)); p += row;
+    if (h->has_h) { HIPCHK(h, hipMemcpy(hr, p, row, hipMemcpyHostToDevice)); p += row; }
+    HIPCHK(h, hipMemcpy(gr + row, p, brow, hipMemcpyHostToDevice)); p += brow;
+    if (h->has_h) { HIPCHK(h, hipMemcpy(hr + row, p, brow, hipMemcpyHostToDevice)); p += brow; }
+    if (h->line_ok) {
+        image_rows(h, gr, h->gb[h->cur], 0);
+        if (h->has_h) image_rows(h, hr, h->hb[h->cur], 0);
+        HIPCHK(h, hipGetLastError());
+        HIPCHK(h, hipStreamSynchronize(h->stream));
+    }
     const size_t nc = h->nc;
     HIPCHK(h, hipMemcpy(h->crho, p, 8 * nc, hipMemcpyHostToDevice)); p += 8 * nc;
     HIPCHK(h, hipMemcpy(h->cU, p, 24 * nc, hipMemcpyHostToDevice)); p += 24 * nc;
@@ -3355,7 +3754,7 @@ int dugks_last_step_ms(dugks_engine *h, double *ms)
 int dugks_set_autotune(dugks_engine *h, int32_t on)
 {
     if (!h) return DUGKS_ERR_INVALID;
-    h->tuning = on ? 1 : 0;
+    h->tuning = on && !use_lines(h) ? 1 : 0;   // the column kernels have one shape
     h->tune_i = -1;
     h->tune_tf.clear();
     h->tune_tc.clear();
@@ -3380,9 +3779,11 @@ int dugks_autotune_steps_left(dugks_engine *h, int32_t *steps)
 int dugks_get_cell_launch(dugks_engine *h, int32_t *nt, int32_t *nib, int32_t *n_blocks)
 {
     if (!h) return DUGKS_ERR_INVALID;
-    if (nt) *nt = h->ntc;
-    if (nib) *nib = h->nibc;
-    if (n_blocks) *n_blocks = h->nvbc;
+    // column kernels: 64 lanes over every iteration of the row
+    const bool lines = use_lines(h);
+    if (nt) *nt = lines ? 64 : h->ntc;
+    if (nib) *nib = lines ? h->nvp / 64 : h->nibc;
+    if (n_blocks) *n_blocks = lines ? 1 : h->nvbc;
     return 0;
 }
 
@@ -3421,9 +3822,10 @@ int dugks_set_face_values(dugks_engine *h, int32_t on)
 int dugks_get_launch(dugks_engine *h, int32_t *nt, int32_t *nib, int32_t *n_blocks, int32_t *nv_padded)
 {
     if (!h) return DUGKS_ERR_INVALID;
-    if (nt) *nt = h->nt;
-    if (nib) *nib = h->nib;
-    if (n_blocks) *n_blocks = h->nvb;
+    const bool lines = use_lines(h);
+    if (nt) *nt = lines ? 64 : h->nt;
+    if (nib) *nib = lines ? h->nvp / 64 : h->nib;
+    if (n_blocks) *n_blocks = lines ? 1 : h->nvb;
     if (nv_padded) *nv_padded = h->nvp;
     return 0;
 }

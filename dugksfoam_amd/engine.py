@@ -222,8 +222,9 @@ class Engine:
         return out, n.value
 
     def face_mfma(self) -> bool:
-        """True when the face moments of non-wall faces are FP64 matrix products
-        (k_face_moments_mx: face-value mode, DUGKS_FACE_MFMA not 0)."""
+        """True in face-value mode with DUGKS_FACE_MFMA not 0: cells of up to 6 faces (4 in 2-D)
+        take the column kernels, which sum the face moments as they form the face values; with
+        more faces the moments of non-wall faces are FP64 matrix products (k_face_moments_mx)."""
         return self._face_mfma and self.face_values()
 
     def fused_cell(self) -> bool:

@@ -197,7 +197,9 @@ int dugks_set_graphs(dugks_engine* h, int32_t on);
  * one warm-up step; every candidate in two rounds), timed with HIP events, then keep the one
  * with the shortest time of each.  The steps are
  * real steps of the simulation; the candidates differ only in how velocity sums are split,
- * i.e. in round-off.  dugks_get_launch / dugks_get_cell_launch report the shapes in use. */
+ * i.e. in round-off.  The kernels over velocity columns (cells of up to 6 faces, 4 in 2-D, in
+ * face-value mode) have one shape set by a rule: nothing is tuned there.
+ * dugks_get_launch / dugks_get_cell_launch report the shapes in use. */
 int dugks_set_autotune(dugks_engine* h, int32_t on);
 /* Steps still to run before the tuning started by dugks_set_autotune ends (0 when idle). */
 int dugks_autotune_steps_left(dugks_engine* h, int32_t* steps);
