@@ -24,11 +24,12 @@
 //              objective seed; S6 face macros; S4/S3 wall: rho_w = out / in, incoming rho_w M(T_w)
 //              -> dJ/dT_w and the outgoing face values
 //   recon_adj  S2 upwind reconstruction -> gbar+ and the gradient; S2 new G = n . grad
-//   grad_adj   least-squares gradient -> gbar+ and the lagged rows G^n
-//   s1_adj     S1 gbar+ = (1 - r) g~ + r geq(M) -> g~^n and M^n; M^n = m(g~^n) folded into g~^n
+//   grad_s1_adj  least-squares gradient -> gbar+ and the lagged rows G^n; S1 gbar+ = (1 - r) g~ + r geq(M) -> g~^n and M^n; M^n = m(g~^n) folded into g~^n
 #pragma once
 
 #include <cmath>
+#include <cstddef>
+#include <type_traits>
 
 #ifdef __HIPCC__
 #define ADJ_HD __host__ __device__ inline
@@ -61,25 +62,70 @@ ADJ_HD bool far_kind(int fk) { return fk == FK_FAR || fk == FK_PIN || fk == FK_P
 // Mirror planes: the incoming value of a velocity is the outgoing value of its mirror.
 ADJ_HD bool mirror_kind(int fk) { return fk == FK_SYM || fk == FK_SPL; }
 
+// An array that no kernel writes while it reads it.  On the device its elements come from the constant
+// address space: those of a point (uniform over the workgroup) are scalar loads, hoisted out of the
+// loops over velocities, where the stores of a loop would have them loaded again by every lane.
+template <class T>
+struct CP {
+    const T *p = nullptr;
+    CP &operator=(const T *q)
+    {
+        p = q;
+        return *this;
+    }
+    explicit operator bool() const { return p != nullptr; }
+    ADJ_HD CP operator+(size_t n) const
+    {
+        CP r;
+        r.p = p + n;
+        return r;
+    }
+    ADJ_HD T operator[](size_t i) const
+    {
+#if defined(__HIP_DEVICE_COMPILE__)
+        return ((const __attribute__((address_space(4))) T *)p)[i];
+#else
+        return p[i];
+#endif
+    }
+};
+
+// Rows of a point's velocities on chip (the phases that pass over them again would read them back through
+// the L2, and a forward step whose reverse does not follow need not write its face values at all; 16000
+// faces of 32^2 velocities: k_face 467 -> 306 us with the scalar loads of CP and one upwind row, k_face_adj
+// 374 -> 294): an executor with local_rows keeps row i (nv values, each
+// written and read by the worker that owns its velocity) there, others in the given work array.
+template <class X, class = void>
+struct has_rows : std::false_type {};
+template <class X>
+struct has_rows<X, std::enable_if_t<X::local_rows>> : std::true_type {};
+
+template <class X>
+ADJ_HD double *row_of(X &x, int i, int nv, double *work)
+{
+    if constexpr (has_rows<X>::value) return x.row(i, nv);
+    else return work;
+}
+
 // Mesh, velocity set and gas; every array is indexed by global face / cell numbers.
 struct AP {
     int D, K, nc, nfi, nf, nv;
     double R, omega, Tref, mu, Pr, kc, dt;   // kc = K + 3 - D
-    const int *cstart, *cface;   // faces of each cell in ascending order
-    const int *owner, *nei;      // nei: internal faces
-    const int *fkind;            // FK_*
-    const int *partner, *pcell;  // cyclic faces: the coupled face and its owner cell
-    const double *S, *Cf, *C, *V, *wf;   // wf: surfaceInterpolation weights
-    const double *pvec, *nvec;   // least-squares vectors [nf][3], [nfi][3]
-    const double *nhat, *adel;   // walls: Sf/|Sf|, 1/deltaCoeffs
-    const double *xi, *wv;       // [nv][3], [nv], reference order
-    const double *Tw, *Uw;       // walls, fixed and far-field faces: T [nf]; walls, fixed: U [nf][3]
-    const double *rb;            // fixed and far-field faces: rho_b [nf]
-    const double *win, *dwin;    // walls: inComingByRho and its T_w derivative
-    const double *pb;            // pressure faces: p_b [nf]
-    const double *muc;           // muRef of each cell's case [nc] (faces: the owner's)
-    const int *sax;              // symmetry faces: the mirror axis [nf]
-    const int *mir;              // [3][nv]: the velocity mirrored across axis a
+    CP<int> cstart, cface;   // faces of each cell in ascending order
+    CP<int> owner, nei;      // nei: internal faces
+    CP<int> fkind;            // FK_*
+    CP<int> partner, pcell;  // cyclic faces: the coupled face and its owner cell
+    CP<double> S, Cf, C, V, wf;   // wf: surfaceInterpolation weights
+    CP<double> pvec, nvec;   // least-squares vectors [nf][3], [nfi][3]
+    CP<double> nhat, adel;   // walls: Sf/|Sf|, 1/deltaCoeffs
+    CP<double> xi, wv;       // [nv][3], [nv], reference order
+    CP<double> Tw, Uw;       // walls, fixed and far-field faces: T [nf]; walls, fixed: U [nf][3]
+    CP<double> rb;            // fixed and far-field faces: rho_b [nf]
+    CP<double> win, dwin;    // walls: inComingByRho and its T_w derivative
+    CP<double> pb;            // pressure faces: p_b [nf]
+    CP<double> muc;           // muRef of each cell's case [nc] (faces: the owner's)
+    CP<int> sax;              // symmetry faces: the mirror axis [nf]
+    CP<int> mir;              // [3][nv]: the velocity mirrored across axis a
 };
 
 // One state: g, h [nc][nv]; Gg, Gh [nf - nfi][nv]; mac [nc][8] = rho, U[3], T, q[3].
@@ -94,7 +140,8 @@ struct FaceRec {
 static_assert(sizeof(FaceRec) == 32 * sizeof(double), "face record");
 
 // xi . S = (x Sx + y Sy) + z Sz without contraction (the upwind test must see exact zeros)
-ADJ_HD double sdot(const double *a, const double *b)
+template <class A, class B>
+ADJ_HD double sdot(const A &a, const B &b)
 {
 #pragma clang fp contract(off)
     return (a[0] * b[0] + a[1] * b[1]) + a[2] * b[2];
@@ -107,6 +154,7 @@ ADJ_HD double tau_of(const AP &p, double mu, double rho, double T)
 
 struct Eq {
     double rho, U[3], T, q[3], RT, pre, k5;   // pre = rho / (2 pi R T)^(D/2), k5 = 1 / (5 rho (RT)^2)
+    double irho, iT, iRT;                     // 1 / rho, 1 / T, 1 / RT
 };
 
 ADJ_HD void eq_set(const AP &p, double rho, const double *U, double T, const double *q, Eq &e)
@@ -120,10 +168,14 @@ ADJ_HD void eq_set(const AP &p, double rho, const double *U, double T, const dou
     e.RT = p.R * T;
     e.pre = rho / pow(sqrt(2.0 * PI * e.RT), (double)p.D);
     e.k5 = 1.0 / (5.0 * rho * e.RT * e.RT);
+    e.irho = 1.0 / rho;
+    e.iT = 1.0 / T;
+    e.iRT = 1.0 / e.RT;
 }
 
 // Shakhov equilibrium, discreteVelocity.C:1016-1044
-ADJ_HD void shakhov(const AP &p, const Eq &e, const double *xi, double &geq, double &heq)
+template <class V>
+ADJ_HD void shakhov(const AP &p, const Eq &e, const V &xi, double &geq, double &heq)
 {
     const double u[3] = {e.U[0] - xi[0], e.U[1] - xi[1], e.U[2] - xi[2]};
     const double c2 = (u[0] * u[0] + u[1] * u[1] + u[2] * u[2]) / e.RT;
@@ -134,11 +186,13 @@ ADJ_HD void shakhov(const AP &p, const Eq &e, const double *xi, double &geq, dou
     heq = (p.kc + P1 * cq * ((c2 - p.D) * p.kc - 2.0 * p.K)) * gB * e.RT;
 }
 
-// acc[0..8) += a d(geq)/d(rho, U, T, q) + b d(heq)/d(rho, U, T, q)
-ADJ_HD void shakhov_vjp(const AP &p, const Eq &e, const double *xi, double a, double b, double *acc)
+// acc[0..8) += a d(geq)/d(rho, U, T, q) + b d(heq)/d(rho, U, T, q); divisions by the point's own values
+// are products with their reciprocals
+template <class V>
+ADJ_HD void shakhov_vjp(const AP &p, const Eq &e, const V &xi, double a, double b, double *acc)
 {
     const double u[3] = {e.U[0] - xi[0], e.U[1] - xi[1], e.U[2] - xi[2]};
-    const double RT = e.RT, T = e.T, rho = e.rho;
+    const double RT = e.RT;
     const double c2 = (u[0] * u[0] + u[1] * u[1] + u[2] * u[2]) / RT;
     const double cq = -(u[0] * e.q[0] + u[1] * e.q[1] + u[2] * e.q[2]) * e.k5;
     const double gB = e.pre * exp(-0.5 * c2);
@@ -146,19 +200,19 @@ ADJ_HD void shakhov_vjp(const AP &p, const Eq &e, const double *xi, double a, do
     const double D = p.D, kc = p.kc, K2 = 2.0 * p.K;
     const double Ag = 1.0 + P1 * cq * (c2 - D - 2.0);
     const double Ah = kc + P1 * cq * ((c2 - D) * kc - K2);
-    const double X = a * Ag + b * RT * Ah;                       // multiplies d(gB)
-    const double Y1 = a * (c2 - D - 2.0) + b * RT * ((c2 - D) * kc - K2);   // multiplies d(cq)
-    const double Y2 = a + b * RT * kc;                           // multiplies cq d(c2)
-    const double gp = gB * P1;
-    acc[0] += gp * (-cq / rho) * Y1 + X * gB / rho;
-    for (int d = 0; d < 3; ++d)
-        acc[1 + d] += gp * (-e.q[d] * e.k5 * Y1 + cq * (2.0 * u[d] / RT) * Y2) - X * gB * u[d] / RT;
-    acc[4] += gp * ((-2.0 * cq / T) * Y1 - cq * (c2 / T) * Y2) + X * gB * (c2 - D) / (2.0 * T) + b * Ah * gB * p.R;
-    for (int d = 0; d < 3; ++d) acc[5 + d] += gp * (-u[d] * e.k5) * Y1;
+    const double X = (a * Ag + b * RT * Ah) * gB;                                      // d(ln gB)
+    const double Y1 = (a * (c2 - D - 2.0) + b * RT * ((c2 - D) * kc - K2)) * gB * P1;   // d(cq)
+    const double Y2 = (a + b * RT * kc) * gB * P1 * cq;                                // d(c2)
+    const double Z = (2.0 * Y2 - X) * e.iRT;
+    acc[0] += (X - cq * Y1) * e.irho;
+    for (int d = 0; d < 3; ++d) acc[1 + d] += u[d] * Z - e.q[d] * e.k5 * Y1;
+    acc[4] += (0.5 * X * (c2 - D) - 2.0 * cq * Y1 - c2 * Y2) * e.iT + b * Ah * gB * p.R;
+    for (int d = 0; d < 3; ++d) acc[5 + d] -= u[d] * e.k5 * Y1;
 }
 
 // equilibriumMaxwellByRho (discreteVelocity.C:1063-1075) and its T derivative
-ADJ_HD double maxwell(const AP &p, const double *U, double T, const double *xi, double &dMdT)
+template <class W, class V>
+ADJ_HD double maxwell(const AP &p, const W &U, double T, const V &xi, double &dMdT)
 {
     const double u[3] = {U[0] - xi[0], U[1] - xi[1], U[2] - xi[2]};
     const double u2 = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
@@ -196,7 +250,8 @@ struct Mom {
     double rho, U[3], T, tau, F, c0, qh[3], A0, P[3][3];
 };
 
-ADJ_HD void mom_acc(double *s, const double *xi, double w, const double *U, double g, double h)
+template <class V>
+ADJ_HD void mom_acc(double *s, const V &xi, double w, const double *U, double g, double h)
 {
     const double c[3] = {xi[0] - U[0], xi[1] - U[1], xi[2] - U[2]};
     const double cc = c[0] * c[0] + c[1] * c[1] + c[2] * c[2];
@@ -256,7 +311,8 @@ ADJ_HD void macro_adj(const AP &p, const Mom &m, const double *ad, double tau_ex
     ga = 0.5 * Tt / den;
 }
 
-ADJ_HD void macro_apply(const double *xi, double w, const double *U, double al, const double *be, double ga,
+template <class V>
+ADJ_HD void macro_apply(const V &xi, double w, const double *U, double al, const double *be, double ga,
                         const double *de, double &ag, double &ah)
 {
     const double c[3] = {xi[0] - U[0], xi[1] - U[1], xi[2] - U[2]};
@@ -275,7 +331,8 @@ ADJ_HD void load_grad(const AP &p, const double *G, int c, int k, double *v)
     for (int d = 0; d < 3; ++d) v[d] = d < p.D ? G[((size_t)c * p.D + d) * p.nv + k] : 0.0;
 }
 
-ADJ_HD double dot3(const double *a, const double *b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; }
+template <class A, class B>
+ADJ_HD double dot3(const A &a, const B &b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; }
 
 // ---------------------------------------------------------------------------------------------
 // Forward step
@@ -310,9 +367,9 @@ template <class X>
 ADJ_HD void wall_in(X &x, const AP &p, int f, double *win, double *dwin)
 {
     double a[2] = {0.0, 0.0};
-    const double *S = p.S + 3 * f;
+    const auto S = p.S + 3 * (size_t)f;
     x.for_k(p.nv, [&](int k) {
-        const double *xi = p.xi + 3 * k;
+        const auto xi = p.xi + 3 * (size_t)k;
         const double s = sdot(xi, S);
         if (s < 0) {
             double dM;
@@ -350,7 +407,7 @@ ADJ_HD void s1_cell(X &x, const AP &p, St s, int c, double *gp, double *hp)
     eq_set(p, rho, U, T, q, e);
     x.for_k(p.nv, [&](int k) {
         double geq, heq;
-        shakhov(p, e, p.xi + 3 * k, geq, heq);
+        shakhov(p, e, p.xi + 3 * (size_t)k, geq, heq);
         const size_t i = ix(c, p.nv, k);
         gp[i] = (1.0 - r) * s.g[i] + r * geq;
         hp[i] = (1.0 - r) * s.h[i] + r * heq;
@@ -370,7 +427,7 @@ ADJ_HD void grad_cell(X &x, const AP &p, St s, int c, const double *gp, const do
         double G[3] = {0, 0, 0}, H[3] = {0, 0, 0};
         for (int e = p.cstart[c]; e < p.cstart[c + 1]; ++e) {
             const int f = p.cface[e];
-            const double *L;
+            CP<double> L;
             double dg, dh;
             if (f < nfi) {
                 const bool own = p.owner[f] == c;
@@ -417,13 +474,36 @@ ADJ_HD void face_value(const AP &p, int f, int k, double s, const double *gp, co
                        const double *gh, double &g, double &h)
 {
     const int nv = p.nv, P = p.owner[f], fk = f < p.nfi ? FK_INTERNAL : p.fkind[f];
-    const double *xi = p.xi + 3 * k, *Cf = p.Cf + 3 * f;
+    const auto xi = p.xi + 3 * (size_t)k, Cf = p.Cf + 3 * (size_t)f;
     const double hx[3] = {0.5 * xi[0] * p.dt, 0.5 * xi[1] * p.dt, 0.5 * xi[2] * p.dt};
+    if (fk == FK_INTERNAL) {
+        // one reconstruction, of the lane's upwind cell, so that a wave with both signs loads no row
+        // that half of it drops; the mean of both where |xi.S| < VSMALL
+        const int N = p.nei[f];
+        const bool own = s >= VSMALL;
+        auto recon = [&](bool o, double &gu, double &hu) {
+            const int u = o ? P : N;
+            double G[3], H[3], d[3];
+            load_grad(p, gg, u, k, G);
+            load_grad(p, gh, u, k, H);
+            for (int q = 0; q < 3; ++q) d[q] = Cf[q] - (o ? p.C[3 * (size_t)P + q] : p.C[3 * (size_t)N + q]) - hx[q];
+            gu = gp[ix(u, nv, k)] + dot3(G, d);
+            hu = hp[ix(u, nv, k)] + dot3(H, d);
+        };
+        recon(own, g, h);
+        if (!own && !(s < -VSMALL)) {
+            double gP, hP;
+            recon(true, gP, hP);
+            g = 0.5 * (g + gP);
+            h = 0.5 * (h + hP);
+        }
+        return;
+    }
     double GP[3], HP[3];
     load_grad(p, gg, P, k, GP);
     load_grad(p, gh, P, k, HP);
-    const double *CP = p.C + 3 * P;
-    const double dO[3] = {Cf[0] - CP[0] - hx[0], Cf[1] - CP[1] - hx[1], Cf[2] - CP[2] - hx[2]};
+    const auto CPc = p.C + 3 * (size_t)P;
+    const double dO[3] = {Cf[0] - CPc[0] - hx[0], Cf[1] - CPc[1] - hx[1], Cf[2] - CPc[2] - hx[2]};
     if (fk == FK_ZG) {
         g = gp[ix(P, nv, k)];   // patchInternalField (discreteVelocity.C:551-555)
         h = hp[ix(P, nv, k)];
@@ -433,12 +513,12 @@ ADJ_HD void face_value(const AP &p, int f, int k, double s, const double *gp, co
         // incoming: the outgoing reconstruction of the mirrored velocity, at its own index
         // (discreteVelocity.C:746-790); xi.S == 0 mirrors onto itself
         const int km = p.mir[p.sax[f] * nv + k];
-        const double *xm = p.xi + 3 * km;
+        const auto xm = p.xi + 3 * (size_t)km;
         const double hm[3] = {0.5 * xm[0] * p.dt, 0.5 * xm[1] * p.dt, 0.5 * xm[2] * p.dt};
         double GM[3], HM[3];
         load_grad(p, gg, P, km, GM);
         load_grad(p, gh, P, km, HM);
-        const double dM[3] = {Cf[0] - CP[0] - hm[0], Cf[1] - CP[1] - hm[1], Cf[2] - CP[2] - hm[2]};
+        const double dM[3] = {Cf[0] - CPc[0] - hm[0], Cf[1] - CPc[1] - hm[1], Cf[2] - CPc[2] - hm[2]};
         g = gp[ix(P, nv, km)] + dot3(GM, dM);
         h = hp[ix(P, nv, km)] + dot3(HM, dM);
         return;
@@ -447,28 +527,6 @@ ADJ_HD void face_value(const AP &p, int f, int k, double s, const double *gp, co
     if (fk == FK_WALL || fk == FK_FIXED || mirror_kind(fk) || far_kind(fk)) {
         g = gP;
         h = hP;
-        return;
-    }
-    if (fk == FK_INTERNAL) {
-        if (s >= VSMALL) {
-            g = gP;
-            h = hP;
-            return;
-        }
-        const int N = p.nei[f];
-        double GN[3], HN[3];
-        load_grad(p, gg, N, k, GN);
-        load_grad(p, gh, N, k, HN);
-        const double *CN = p.C + 3 * N;
-        const double dN[3] = {Cf[0] - CN[0] - hx[0], Cf[1] - CN[1] - hx[1], Cf[2] - CN[2] - hx[2]};
-        const double gN = gp[ix(N, nv, k)] + dot3(GN, dN), hN = hp[ix(N, nv, k)] + dot3(HN, dN);
-        if (s < -VSMALL) {
-            g = gN;
-            h = hN;
-        } else {
-            g = 0.5 * (gN + gP);
-            h = 0.5 * (hN + hP);
-        }
         return;
     }
     // cyclic: coupled value w phi_P + (1 - w) phi_N and gradient, at distance -hx
@@ -498,62 +556,64 @@ ADJ_HD void face_value(const AP &p, int f, int k, double s, const double *gp, co
 }
 
 // S2-S7 of one face: face values (S2), Maxwell wall density and incoming values (S3, S4), face
-// macros (S6) and, when gr is given, the relaxed face values (S7).  jacc[f] += c_f (rho U)_f . S_f
-// when jacc is given.
+// macros (S6) and, when gr is given, the relaxed face values (S7).  The face values end in gf, hf when
+// keep is set (the reverse sweep reads them); otherwise these are work arrays.  jacc[f] += c_f (rho U)_f
+// . S_f when jacc is given.
 template <class X>
 ADJ_HD void face_fwd(X &x, const AP &p, int f, const double *mac, const double *gp, const double *hp,
-                     const double *gg, const double *gh, double *gf, double *hf, FaceRec *fr, double *gr,
+                     const double *gg, const double *gh, double *gf, double *hf, bool keep, FaceRec *fr, double *gr,
                      double *hr, const double *coef, double *jacc)
 {
     const int nv = p.nv, fk = f < p.nfi ? FK_INTERNAL : p.fkind[f];
-    const double *S = p.S + 3 * f;
-    double out[1] = {0.0};
-    x.for_k(nv, [&](int k) {
-        const double s = sdot(p.xi + 3 * k, S);
-        if (maxwell_kind(fk) && !(s > 0)) return;
-        double g, h;
-        face_value(p, f, k, s, gp, hp, gg, gh, g, h);
-        gf[ix(f, nv, k)] = g;
-        hf[ix(f, nv, k)] = h;
-        if (fk == FK_WALL) out[0] += p.wv[k] * s * g;
-    });
-    double rho_w = 0.0;
-    if (fk == FK_WALL) {
-        x.template sum<1>(out);
-        rho_w = out[0] / p.win[f];   // calculatedMaxwell evaluate (cMaxwell.C:139-164)
-        const double Tw = p.Tw[f];
-        x.for_k(nv, [&](int k) {
-            const double *xi = p.xi + 3 * k;
-            if (sdot(xi, S) > 0) return;
-            double dM;
-            const double g = rho_w * maxwell(p, p.Uw + 3 * f, Tw, xi, dM);
-            gf[ix(f, nv, k)] = g;
-            hf[ix(f, nv, k)] = g * (p.R * Tw) * p.kc;
-        });
-    }
-    if (fk == FK_FIXED || far_kind(fk)) {
-        // incoming rho_b M(U, T_b): fixed faces freeze U_b (discreteVelocity.C:312-344, 556-573),
-        // far-field faces take the owner cell's velocity (discreteVelocity.C:588-602)
-        double Tb = p.Tw[f], rb = p.rb[f];
-        if (far_kind(fk)) far_bc(p, f, fk, mac, rb, Tb);
-        const double *Ub = far_kind(fk) ? mac + 8 * (size_t)p.owner[f] + 1 : p.Uw + 3 * f;
-        x.for_k(nv, [&](int k) {
-            const double *xi = p.xi + 3 * k;
-            if (sdot(xi, S) > 0) return;
-            double dM;
-            const double g = rb * maxwell(p, Ub, Tb, xi, dM);
-            gf[ix(f, nv, k)] = g;
-            hf[ix(f, nv, k)] = g * (p.R * Tb) * p.kc;
-        });
-    }
+    const auto S = p.S + 3 * (size_t)f;
+    const size_t f0 = ix(f, nv, 0);
+    double *rg = row_of(x, 0, nv, gf + f0), *rh = row_of(x, 1, nv, hf + f0);
+    const bool store = has_rows<X>::value && keep;
     double a[5] = {0, 0, 0, 0, 0};
-    x.for_k(nv, [&](int k) {
-        const double *xi = p.xi + 3 * k;
-        const double w = p.wv[k], g = gf[ix(f, nv, k)], h = hf[ix(f, nv, k)];
+    // a face value, and its part of rho, rho U, rho E
+    auto put = [&](int k, double g, double h) {
+        const auto xi = p.xi + 3 * (size_t)k;
+        const double w = p.wv[k];
+        rg[k] = g;
+        rh[k] = h;
+        if (store) {
+            gf[f0 + k] = g;
+            hf[f0 + k] = h;
+        }
         a[0] += w * g;
         for (int d = 0; d < 3; ++d) a[1 + d] += w * g * xi[d];
         a[4] += 0.5 * w * (g * dot3(xi, xi) + h);
+    };
+    double out[1] = {0.0};
+    x.for_k(nv, [&](int k) {
+        const double s = sdot(p.xi + 3 * (size_t)k, S);
+        if (maxwell_kind(fk) && !(s > 0)) return;
+        double g, h;
+        face_value(p, f, k, s, gp, hp, gg, gh, g, h);
+        put(k, g, h);
+        if (fk == FK_WALL) out[0] += p.wv[k] * s * g;
     });
+    double rho_w = 0.0;
+    if (maxwell_kind(fk)) {
+        // incoming rho_b M(U, T_b): walls take rho_w from their outgoing flux, fixed faces freeze U_b
+        // (discreteVelocity.C:312-344, 556-573), far-field faces take the owner cell's velocity
+        // (discreteVelocity.C:588-602)
+        double Tb = p.Tw[f], rb = p.rb[f];
+        if (fk == FK_WALL) {
+            x.template sum<1>(out);
+            rb = rho_w = out[0] / p.win[f];   // calculatedMaxwell evaluate (cMaxwell.C:139-164)
+        }
+        if (far_kind(fk)) far_bc(p, f, fk, mac, rb, Tb);
+        double Ub[3];
+        for (int d = 0; d < 3; ++d) Ub[d] = far_kind(fk) ? mac[8 * (size_t)p.owner[f] + 1 + d] : p.Uw[3 * (size_t)f + d];
+        x.for_k(nv, [&](int k) {
+            const auto xi = p.xi + 3 * (size_t)k;
+            if (sdot(xi, S) > 0) return;
+            double dM;
+            const double g = rb * maxwell(p, Ub, Tb, xi, dM);
+            put(k, g, g * (p.R * Tb) * p.kc);
+        });
+    }
     x.template sum<5>(a);
     Mom m;
     m.rho = a[0];
@@ -561,7 +621,7 @@ ADJ_HD void face_fwd(X &x, const AP &p, int f, const double *mac, const double *
     m.T = (a[4] - 0.5 * m.rho * dot3(m.U, m.U)) / ((p.K + 3) / 2.0 * p.R * m.rho);
     m.tau = tau_of(p, p.muc[p.owner[f]], m.rho, m.T);
     double sm[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    x.for_k(nv, [&](int k) { mom_acc(sm, p.xi + 3 * k, p.wv[k], m.U, gf[ix(f, nv, k)], hf[ix(f, nv, k)]); });
+    x.for_k(nv, [&](int k) { mom_acc(sm, p.xi + 3 * (size_t)k, p.wv[k], m.U, rg[k], rh[k]); });
     x.template sum<10>(sm);
     mom_set(m, sm);
     const double hdt = 0.5 * p.dt;
@@ -591,37 +651,41 @@ ADJ_HD void face_fwd(X &x, const AP &p, int f, const double *mac, const double *
     Eq e;
     eq_set(p, m.rho, m.U, m.T, q, e);
     x.for_k(nv, [&](int k) {
-        const double *xi = p.xi + 3 * k;
-        const size_t i = ix(f, nv, k);
-        const bool out = sdot(xi, S) > 0;
-        if (open_kind(fk) && fk != FK_SPL && !out) {
-            gr[i] = gf[i];   // incoming halves are not relaxed (their patch operators are no-ops, *Fvs.H:161-181)
-            hr[i] = hf[i];
-            return;
+        const auto xi = p.xi + 3 * (size_t)k;
+        const bool outgoing = sdot(xi, S) > 0;
+        double g = rg[k], h = rh[k];
+        // incoming halves are not relaxed (their patch operators are no-ops, *Fvs.H:161-181)
+        if (!open_kind(fk) || fk == FK_SPL || outgoing) {
+            double geq, heq;
+            shakhov(p, e, xi, geq, heq);
+            g = (1.0 - r) * g + r * geq;
+            h = (1.0 - r) * h + r * heq;
+            if (fk == FK_SPL && outgoing) {
+                // symmetryPlane: the field operation relaxed every value (discreteVelocity.C:880-881),
+                // the loop over non-coupled patches relaxes the outgoing ones again (905-920)
+                g = (1.0 - r) * g + r * geq;
+                h = (1.0 - r) * h + r * heq;
+            }
         }
-        double geq, heq;
-        shakhov(p, e, xi, geq, heq);
-        gr[i] = (1.0 - r) * gf[i] + r * geq;
-        hr[i] = (1.0 - r) * hf[i] + r * heq;
-        if (fk == FK_SPL && out) {
-            // symmetryPlane: the field operation relaxed every value (discreteVelocity.C:880-881),
-            // the loop over non-coupled patches relaxes the outgoing ones again (905-920)
-            gr[i] = (1.0 - r) * gr[i] + r * geq;
-            hr[i] = (1.0 - r) * hr[i] + r * heq;
-        }
+        gr[f0 + k] = g;
+        hr[f0 + k] = h;
     });
 }
 
-// S8 (discreteVelocity.C:934-978) and S9 (fvDVM.C:597-728) of one cell into state nx
+// S8 (discreteVelocity.C:934-978) and S9 (fvDVM.C:597-728) of one cell into state nx; with s1 also S1
+// of the next step, over this step's gbar+ of the cell, from the row that is at hand (8000 cells of 32^2
+// velocities: 201 + 55 us as two kernels, 224 as one; memory bound).
 template <class X>
-ADJ_HD void cell_fwd(X &x, const AP &p, St s, int c, const double *gp, const double *hp, const double *gr,
-                     const double *hr, St nx)
+ADJ_HD void cell_fwd(X &x, const AP &p, St s, int c, double *gp, double *hp, const double *gr, const double *hr,
+                     St nx, bool s1)
 {
     const int nv = p.nv;
+    const size_t c0 = ix(c, nv, 0);
+    double *rg = row_of(x, 0, nv, nx.g + c0), *rh = row_of(x, 1, nv, nx.h + c0);
     const double V = p.V[c], dt = p.dt;
     double a[5] = {0, 0, 0, 0, 0};
     x.for_k(nv, [&](int k) {
-        const double *xi = p.xi + 3 * k;
+        const auto xi = p.xi + 3 * (size_t)k;
         const size_t i = ix(c, nv, k);
         double g = -1.0 / 3 * s.g[i] + 4.0 / 3 * gp[i];
         double h = -1.0 / 3 * s.h[i] + 4.0 / 3 * hp[i];
@@ -637,8 +701,8 @@ ADJ_HD void cell_fwd(X &x, const AP &p, St s, int c, const double *gp, const dou
                 h += fh;
             }
         }
-        nx.g[i] = g;
-        nx.h[i] = h;
+        nx.g[i] = rg[k] = g;
+        nx.h[i] = rh[k] = h;
         const double w = p.wv[k];
         a[0] += w * g;
         for (int d = 0; d < 3; ++d) a[1 + d] += w * g * xi[d];
@@ -651,7 +715,7 @@ ADJ_HD void cell_fwd(X &x, const AP &p, St s, int c, const double *gp, const dou
     const double T = (a[4] - 0.5 * rho * dot3(U, U)) / ((p.K + 3) / 2.0 * p.R * rho);
     const double tau = tau_of(p, p.muc[c], rho, T);
     double sm[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    x.for_k(nv, [&](int k) { mom_acc(sm, p.xi + 3 * k, p.wv[k], U, nx.g[ix(c, nv, k)], nx.h[ix(c, nv, k)]); });
+    x.for_k(nv, [&](int k) { mom_acc(sm, p.xi + 3 * (size_t)k, p.wv[k], U, rg[k], rh[k]); });
     x.template sum<10>(sm);
     const double F = 2.0 * tau / (2.0 * tau + dt * p.Pr);   // fvDVM.C:727
     if (x.leader()) {
@@ -663,6 +727,16 @@ ADJ_HD void cell_fwd(X &x, const AP &p, St s, int c, const double *gp, const dou
         }
         m[4] = T;
     }
+    if (!s1) return;
+    const double r = 1.5 * dt / (2.0 * tau + dt), q[3] = {F * sm[0], F * sm[1], F * sm[2]};
+    Eq e;
+    eq_set(p, rho, U, T, q, e);
+    x.for_k(nv, [&](int k) {
+        double geq, heq;
+        shakhov(p, e, p.xi + 3 * (size_t)k, geq, heq);
+        gp[c0 + k] = (1.0 - r) * rg[k] + r * geq;
+        hp[c0 + k] = (1.0 - r) * rh[k] + r * heq;
+    });
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -678,45 +752,47 @@ ADJ_HD void face_adj(X &x, const AP &p, int f, const double *mac, const FaceRec 
                      double *abh, double *dTw, double *aUf)
 {
     const int nv = p.nv, fk = f < p.nfi ? FK_INTERNAL : p.fkind[f];
-    const double *S = p.S + 3 * f;
-    const FaceRec &R = fr[f];
+    const auto S = p.S + 3 * (size_t)f;
+    const FaceRec R = fr[f];
+    const size_t f0 = ix(f, nv, 0);
+    // the adjoint of the face values between the passes
+    double *rg = row_of(x, 0, nv, abf + f0), *rh = row_of(x, 1, nv, abh + f0);
     const int P = p.owner[f], N = fk == FK_INTERNAL ? p.nei[f] : -1;
-    const double dt = p.dt, VP = p.V[P], VN = N >= 0 ? p.V[N] : 1.0;
+    // no division inside the loops: one by a uniform value takes as many instructions as a dozen products
+    const double dt = p.dt, dtP = dt / p.V[P], dtN = N >= 0 ? dt / p.V[N] : 0.0;
     const double cf = coef ? coef[f] : 0.0;
     Eq e;
     eq_set(p, R.rho, R.U, R.T, R.q, e);
     double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     x.for_k(nv, [&](int k) {
-        const double *xi = p.xi + 3 * k;
+        const auto xi = p.xi + 3 * (size_t)k;
         const double s = sdot(xi, S);
         const size_t i = ix(f, nv, k);
-        double af = -(s * dt) * ag1[ix(P, nv, k)] / VP, bf = -(s * dt) * ah1[ix(P, nv, k)] / VP;
+        double af = -s * (dtP * ag1[ix(P, nv, k)]), bf = -s * (dtP * ah1[ix(P, nv, k)]);
         if (N >= 0) {
-            af += (s * dt) * ag1[ix(N, nv, k)] / VN;
-            bf += (s * dt) * ah1[ix(N, nv, k)] / VN;
+            af += s * (dtN * ag1[ix(N, nv, k)]);
+            bf += s * (dtN * ah1[ix(N, nv, k)]);
         }
         double ab = af, bb = bf;
-        if (fk == FK_SPL && s > 0) {
-            // two relaxations, g1 = (1 - r) gf + r geq and gr = (1 - r) g1 + r geq
-            double geq, heq;
+        if (!open_kind(fk) || fk == FK_SPL || s > 0) {
+            double geq, heq, we = R.r, left = 1.0 - R.r;
             shakhov(p, e, xi, geq, heq);
-            const double g1 = (1.0 - R.r) * gf[i] + R.r * geq, h1 = (1.0 - R.r) * hf[i] + R.r * heq;
-            acc[0] += af * (geq - g1) + bf * (heq - h1) + (1.0 - R.r) * (af * (geq - gf[i]) + bf * (heq - hf[i]));
-            const double we = R.r * (2.0 - R.r);
+            double a0 = af * (geq - gf[i]) + bf * (heq - hf[i]);
+            if (fk == FK_SPL && s > 0) {
+                // two relaxations, g1 = (1 - r) gf + r geq and gr = (1 - r) g1 + r geq
+                const double g1 = left * gf[i] + R.r * geq, h1 = left * hf[i] + R.r * heq;
+                a0 = af * (geq - g1) + bf * (heq - h1) + left * a0;
+                we = R.r * (2.0 - R.r);
+                left *= left;
+            }
+            acc[0] += a0;
             shakhov_vjp(p, e, xi, we * af, we * bf, acc + 1);
-            ab = (1.0 - R.r) * (1.0 - R.r) * af;
-            bb = (1.0 - R.r) * (1.0 - R.r) * bf;
-        } else if (!open_kind(fk) || fk == FK_SPL || s > 0) {
-            double geq, heq;
-            shakhov(p, e, xi, geq, heq);
-            acc[0] += af * (geq - gf[i]) + bf * (heq - hf[i]);
-            shakhov_vjp(p, e, xi, R.r * af, R.r * bf, acc + 1);
-            ab = (1.0 - R.r) * af;
-            bb = (1.0 - R.r) * bf;
+            ab = left * af;
+            bb = left * bf;
         }
         if (cf != 0.0) ab += cf * p.wv[k] * s;
-        abf[i] = ab;
-        abh[i] = bb;
+        rg[k] = ab;
+        rh[k] = bb;
     });
     x.template sum<9>(acc);
     const double hdt = 0.5 * dt;
@@ -745,17 +821,18 @@ ADJ_HD void face_adj(X &x, const AP &p, int f, const double *mac, const FaceRec 
     double rbf = fk == FK_FIXED || fk == FK_FAR ? p.rb[f] : 0.0;
     if (far_kind(fk)) far_bc(p, f, fk, mac, rbf, Tw);
     const double hfac = p.R * Tw * p.kc;
-    const double *Ub = far_kind(fk) ? mac + 8 * (size_t)p.owner[f] + 1 : p.Uw + 3 * f;
+    double Ub[3] = {0.0, 0.0, 0.0};
+    if (maxwell_kind(fk))
+        for (int d = 0; d < 3; ++d) Ub[d] = far_kind(fk) ? mac[8 * (size_t)p.owner[f] + 1 + d] : p.Uw[3 * (size_t)f + d];
     // walls: M sum, dT; fixed and far-field kinds: dM sum (d rho_b), dT_b, dU of the owner (far)
     double wa[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     x.for_k(nv, [&](int k) {
-        const double *xi = p.xi + 3 * k;
-        const size_t i = ix(f, nv, k);
-        double ab = abf[i], bb = abh[i];
+        const auto xi = p.xi + 3 * (size_t)k;
+        double ab = rg[k], bb = rh[k];
         macro_apply(xi, p.wv[k], m.U, al, be, ga, de, ab, bb);
         if (fk == FK_WALL && !(sdot(xi, S) > 0)) {
             double dM;
-            const double M = maxwell(p, p.Uw + 3 * f, Tw, xi, dM);
+            const double M = maxwell(p, Ub, Tw, xi, dM);
             const double t = ab + bb * hfac;
             wa[0] += t * M;
             wa[1] += t * R.rho_w * dM + bb * R.rho_w * M * p.R * p.kc;
@@ -774,8 +851,13 @@ ADJ_HD void face_adj(X &x, const AP &p, int f, const double *mac, const FaceRec 
             ab = 0.0;
             bb = 0.0;
         }
-        abf[i] = ab;
-        abh[i] = bb;
+        if (fk == FK_WALL) {
+            rg[k] = ab;
+            rh[k] = bb;
+        } else {
+            abf[f0 + k] = ab;
+            abh[f0 + k] = bb;
+        }
     });
     if (fk == FK_FIXED || far_kind(fk)) {
         x.template sum<5>(wa);
@@ -805,9 +887,10 @@ ADJ_HD void face_adj(X &x, const AP &p, int f, const double *mac, const FaceRec 
     const double oh = wa[0] / p.win[f], ih = -wa[0] * R.rho_w / p.win[f];
     if (x.leader()) dTw[f] += wa[1] + ih * p.dwin[f];
     x.for_k(nv, [&](int k) {
-        const double *xi = p.xi + 3 * k;
+        const auto xi = p.xi + 3 * (size_t)k;
         const double s = sdot(xi, S);
-        if (s > 0) abf[ix(f, nv, k)] += oh * p.wv[k] * s;
+        abf[f0 + k] = s > 0 ? rg[k] + oh * p.wv[k] * s : rg[k];
+        abh[f0 + k] = rh[k];
     });
 }
 
@@ -819,9 +902,9 @@ ADJ_HD void recon_adj(X &x, const AP &p, int c, const double *abf, const double 
                       double *agg, double *agh)
 {
     const int nv = p.nv, nfi = p.nfi;
-    const double *Cc = p.C + 3 * c;
+    const auto Cc = p.C + 3 * (size_t)c;
     x.for_k(nv, [&](int k) {
-        const double *xi = p.xi + 3 * k;
+        const auto xi = p.xi + 3 * (size_t)k;
         const double hx[3] = {0.5 * xi[0] * p.dt, 0.5 * xi[1] * p.dt, 0.5 * xi[2] * p.dt};
         const size_t i = ix(c, nv, k);
         double a = 4.0 / 3 * ag1[i], ah = 4.0 / 3 * ah1[i];
@@ -829,7 +912,7 @@ ADJ_HD void recon_adj(X &x, const AP &p, int c, const double *abf, const double 
         for (int e = p.cstart[c]; e < p.cstart[c + 1]; ++e) {
             const int f = p.cface[e];
             const double s = sdot(xi, p.S + 3 * f);
-            const double *Cf = p.Cf + 3 * f;
+            const auto Cf = p.Cf + 3 * (size_t)f;
             const double d[3] = {Cf[0] - Cc[0] - hx[0], Cf[1] - Cc[1] - hx[1], Cf[2] - Cc[2] - hx[2]};
             const double vg = abf[ix(f, nv, k)], vh = abh[ix(f, nv, k)];
             if (f < nfi) {
@@ -907,14 +990,30 @@ ADJ_HD void recon_adj(X &x, const AP &p, int c, const double *abf, const double 
     });
 }
 
-// Reverse of the least-squares gradient gathered at one cell: adds to the adjoint of gbar+ and
-// writes the adjoint of the lagged rows G^n of its wall faces.
+// Reverse of the least-squares gradient gathered at one cell (adds to the adjoint of gbar+, writes the
+// adjoint of the lagged rows G^n of its wall faces), of S1, then the adjoint of the state's macros (S9 of
+// the previous step) folded into the distributions: writes the adjoint of g~^n, h~^n.  One kernel: the
+// adjoint of gbar+ stays on chip between its parts (8000 cells of 32^2 velocities: 231 + 186 -> 292 us, bound
+// by the latency that 3 waves a SIMD leave; held to fewer registers the sums spill, 397 us).
 template <class X>
-ADJ_HD void grad_adj(X &x, const AP &p, int c, const double *agg, const double *agh, double *apg, double *aph,
-                     double *AGg, double *AGh)
+ADJ_HD void grad_s1_adj(X &x, const AP &p, St s, int c, const double *ag1, const double *ah1, const double *agg,
+                        const double *agh, double *apg, double *aph, const double *aUf, double *AGg, double *AGh,
+                        double *ag0, double *ah0)
 {
     const int nv = p.nv, nfi = p.nfi;
+    const size_t c0 = ix(c, nv, 0);
+    // the adjoint of gbar+ between the passes
+    double *rg = row_of(x, 0, nv, apg + c0), *rh = row_of(x, 1, nv, aph + c0);
+    double rho, U[3], T, q[3];
+    cell_macros(p, s.mac + 8 * (size_t)c, rho, U, T, q);
+    const double tau = tau_of(p, p.muc[c], rho, T);
+    const double r = 1.5 * p.dt / (2.0 * tau + p.dt);
+    Eq e;
+    eq_set(p, rho, U, T, q, e);
+    double acc[19];
+    for (int i = 0; i < 19; ++i) acc[i] = 0.0;
     x.for_k(nv, [&](int k) {
+        const auto xi = p.xi + 3 * (size_t)k;
         const size_t i = ix(c, nv, k);
         double a = apg[i], ah = aph[i];
         double Gc[3], Hc[3];
@@ -922,7 +1021,7 @@ ADJ_HD void grad_adj(X &x, const AP &p, int c, const double *agg, const double *
         load_grad(p, agh, c, k, Hc);
         for (int e = p.cstart[c]; e < p.cstart[c + 1]; ++e) {
             const int f = p.cface[e];
-            const double *Lc, *Lo;
+            CP<double> Lc, Lo;
             int o;
             if (f < nfi) {
                 const bool own = p.owner[f] == c;
@@ -947,34 +1046,12 @@ ADJ_HD void grad_adj(X &x, const AP &p, int c, const double *agg, const double *
             a += dot3(Lo, Go) - dot3(Lc, Gc);
             ah += dot3(Lo, Ho) - dot3(Lc, Hc);
         }
-        apg[i] = a;
-        aph[i] = ah;
-    });
-}
-
-// Reverse of S1 at one cell, then the adjoint of the state's macros (S9 of the previous step)
-// folded into the distributions: writes the adjoint of g~^n, h~^n.
-template <class X>
-ADJ_HD void s1_adj(X &x, const AP &p, St s, int c, const double *ag1, const double *ah1, const double *apg,
-                   const double *aph, const double *aUf, double *ag0, double *ah0)
-{
-    const int nv = p.nv;
-    double rho, U[3], T, q[3];
-    cell_macros(p, s.mac + 8 * (size_t)c, rho, U, T, q);
-    const double tau = tau_of(p, p.muc[c], rho, T);
-    const double r = 1.5 * p.dt / (2.0 * tau + p.dt);
-    Eq e;
-    eq_set(p, rho, U, T, q, e);
-    double acc[19];
-    for (int i = 0; i < 19; ++i) acc[i] = 0.0;
-    x.for_k(nv, [&](int k) {
-        const double *xi = p.xi + 3 * k;
-        const size_t i = ix(c, nv, k);
-        const double a = apg[i], b = aph[i];
+        rg[k] = a;
+        rh[k] = ah;
         double geq, heq;
         shakhov(p, e, xi, geq, heq);
-        acc[0] += a * (geq - s.g[i]) + b * (heq - s.h[i]);
-        shakhov_vjp(p, e, xi, r * a, r * b, acc + 1);
+        acc[0] += a * (geq - s.g[i]) + ah * (heq - s.h[i]);
+        shakhov_vjp(p, e, xi, r * a, r * ah, acc + 1);
         mom_acc(acc + 9, xi, p.wv[k], U, s.g[i], s.h[i]);
     });
     x.template sum<19>(acc);
@@ -1001,9 +1078,9 @@ ADJ_HD void s1_adj(X &x, const AP &p, St s, int c, const double *ag1, const doub
     macro_adj(p, m, acc + 1, th, al, be, ga, de);
     x.for_k(nv, [&](int k) {
         const size_t i = ix(c, nv, k);
-        double a = -1.0 / 3 * ag1[i] + (1.0 - r) * apg[i];
-        double b = -1.0 / 3 * ah1[i] + (1.0 - r) * aph[i];
-        macro_apply(p.xi + 3 * k, p.wv[k], U, al, be, ga, de, a, b);
+        double a = -1.0 / 3 * ag1[i] + (1.0 - r) * rg[k];
+        double b = -1.0 / 3 * ah1[i] + (1.0 - r) * rh[k];
+        macro_apply(p.xi + 3 * (size_t)k, p.wv[k], U, al, be, ga, de, a, b);
         ag0[i] = a;
         ah0[i] = b;
     });

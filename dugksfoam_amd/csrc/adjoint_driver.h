@@ -43,8 +43,12 @@ struct k_face {};
 struct k_cell {};
 struct k_face_adj {};
 struct k_recon_adj {};
-struct k_grad_adj {};
-struct k_s1_adj {};
+struct k_grad_s1_adj {};
+
+// The phases that go over a point's velocities more than once, with two rows between the passes.
+template <class Tag>
+struct uses_rows : std::bool_constant<std::is_same_v<Tag, k_face> || std::is_same_v<Tag, k_cell> ||
+                                      std::is_same_v<Tag, k_face_adj> || std::is_same_v<Tag, k_grad_s1_adj>> {};
 
 struct Mesh {
     int D = 0, K = 0, nc = 0, nfi = 0, nf = 0, nv = 0;
@@ -349,8 +353,9 @@ struct Engine {
     FaceRec *fslot_r(int s) const { return reinterpret_cast<FaceRec *>(fslot_g(s) + 2 * nfv); }
 
     // one forward step's phases from state a; with fwd, the new state into b.  The face values
-    // and records go to the work arrays, or to face-tape slot `slot` when it is >= 0.
-    void recompute(St a, St b, int step, bool fwd, bool j, int slot = -1)
+    // and records go to the work arrays, or to face-tape slot `slot` when it is >= 0.  have_s1: gp, hp
+    // hold S1 of a already; next_s1: leave S1 of b there.
+    void recompute(St a, St b, bool fwd, bool j, int slot, bool have_s1, bool next_s1)
     {
         const AP q = p;
         double *gp_ = gp, *hp_ = hp, *gg_ = gg, *gh_ = gh;
@@ -360,18 +365,21 @@ struct Engine {
         const double *cf = coef;
         double *ja = j ? jacc : nullptr;
         double *Gng = fwd ? b.Gg : nullptr, *Gnh = fwd ? b.Gh : nullptr;
-        be.template launch<k_s1>(q.nc, ADJ_FN { s1_cell(x, q, a, i, gp_, hp_); });
+        // a step whose reverse follows, now or from the tape, keeps its face values
+        const bool keep = slot >= 0 || !fwd;
+        if (!have_s1) be.template launch<k_s1>(q.nc, ADJ_FN { s1_cell(x, q, a, i, gp_, hp_); });
         be.template launch<k_grad>(q.nc, ADJ_FN { grad_cell(x, q, a, i, gp_, hp_, gg_, gh_, Gng, Gnh); });
         const double *mac = a.mac;
-        be.template launch<k_face>(q.nf, ADJ_FN { face_fwd(x, q, i, mac, gp_, hp_, gg_, gh_, gf_, hf_, fr_, gr, hr, cf, ja); });
-        if (fwd) be.template launch<k_cell>(q.nc, ADJ_FN { cell_fwd(x, q, a, i, gp_, hp_, gr, hr, b); });
+        be.template launch<k_face>(q.nf, ADJ_FN { face_fwd(x, q, i, mac, gp_, hp_, gg_, gh_, gf_, hf_, keep, fr_, gr, hr, cf, ja); });
+        if (fwd) be.template launch<k_cell>(q.nc, ADJ_FN { cell_fwd(x, q, a, i, gp_, hp_, gr, hr, b, next_s1); });
     }
 
     // reverse of step n (state a = state n); cur: index of the adjoint of state n + 1.  The
-    // step's face values and records come from face-tape slot `slot` (>= 0) or are recomputed.
-    void reverse(St a, int n, bool seed, int &cur, int slot = -1)
+    // step's face values and records come from face-tape slot `slot` (>= 0) or are recomputed (have_s1:
+    // from the S1 that gp, hp hold).
+    void reverse(St a, int n, bool seed, int &cur, int slot, bool have_s1)
     {
-        if (slot < 0) recompute(a, a, n, false, false);
+        if (slot < 0) recompute(a, a, false, false, -1, have_s1, false);
         const AP q = p;
         const FaceRec *fr_ = slot >= 0 ? fslot_r(slot) : fr;
         const double *gf_ = slot >= 0 ? fslot_g(slot) : gf, *hf_ = slot >= 0 ? fslot_h(slot) : hf;
@@ -384,8 +392,9 @@ struct Engine {
         be.template launch<k_face_adj>(q.nf, ADJ_FN { face_adj(x, q, i, mac, fr_, gf_, hf_, ag1, ah1, cf, abf_, abh_, dTw_, aUf_); });
         if (n == 0) return;   // the initial state's adjoint is not needed
         be.template launch<k_recon_adj>(q.nc, ADJ_FN { recon_adj(x, q, i, abf_, abh_, ag1, ah1, AG1g, AG1h, apg_, aph_, agg_, agh_); });
-        be.template launch<k_grad_adj>(q.nc, ADJ_FN { grad_adj(x, q, i, agg_, agh_, apg_, aph_, AG0g, AG0h); });
-        be.template launch<k_s1_adj>(q.nc, ADJ_FN { s1_adj(x, q, a, i, ag1, ah1, apg_, aph_, aUf_, ag0, ah0); });
+        be.template launch<k_grad_s1_adj>(q.nc, ADJ_FN {
+            grad_s1_adj(x, q, a, i, ag1, ah1, agg_, agh_, apg_, aph_, aUf_, AG0g, AG0h, ag0, ah0);
+        });
         cur ^= 1;
     }
 
@@ -454,7 +463,7 @@ struct Engine {
         be.tic(0);
         for (int n = 0; n < nsteps; ++n) {
             if (n % C == 0) copy_state(state(n / C), cur);
-            recompute(cur, nxt, n, true, n + 1 >= first);
+            recompute(cur, nxt, true, n + 1 >= first, -1, n > 0, n + 1 < nsteps);
             std::swap(cur, nxt);
         }
         be.tic(1);
@@ -473,8 +482,9 @@ struct Engine {
             const int n0 = seg * C, n1 = std::min(nsteps, n0 + C);
             auto tape = [&](int n) { return n == n0 ? state(seg) : state(ncp + (n - n0 - 1)); };
             auto slot = [&](int n) { return n + 1 < n1 && n - n0 < ftape_slots ? n - n0 : -1; };
-            for (int n = n0; n + 1 < n1; ++n) recompute(tape(n), tape(n + 1), n, true, false, slot(n));
-            for (int n = n1 - 1; n >= n0; --n) reverse(tape(n), n, n + 1 >= first, ca, slot(n));
+            for (int n = n0; n + 1 < n1; ++n) recompute(tape(n), tape(n + 1), true, false, slot(n), n > n0, true);
+            // the last step's S1 is left by the step before it
+            for (int n = n1 - 1; n >= n0; --n) reverse(tape(n), n, n + 1 >= first, ca, slot(n), n == n1 - 1 && n > n0);
         }
         be.tic(3);
         std::vector<double> dh(m.nf);

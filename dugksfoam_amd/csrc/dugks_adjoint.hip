@@ -19,18 +19,21 @@
 
 #include "../../include/dugks.h"
 #include "adjoint_driver.h"
+#include "lane_sums.h"
 
 namespace {
 
-#ifndef DUGKS_ADJ_NT
-#define DUGKS_ADJ_NT 128
-#endif
-constexpr int NT = DUGKS_ADJ_NT;     // lanes per workgroup (a multiple of the 64-lane wavefront)
-constexpr int SUM_MAX = 32;          // widest workgroup reduction of adjoint_core.h
+constexpr long NT_FILL = 2048;            // half of the device's wave slots at 4 waves a SIMD
+constexpr int SUM_MAX = 32;               // widest workgroup reduction of adjoint_core.h
+constexpr size_t ROWS_MAX = 32 * 1024;   // LDS for the two rows of a workgroup: 5 of them on a CU
 
-// Executor of adjoint_core.h inside a workgroup.
+// Executor of adjoint_core.h inside a workgroup of NT lanes; ROWS: its two rows are in LDS.
+template <int NT, bool ROWS>
 struct GX {
-    double *lds;
+    static constexpr bool local_rows = ROWS;
+    double *lds, *rows;
+
+    __host__ __device__ double *row(int i, int nv) { return rows + (size_t)i * nv; }
 
     template <class F>
     __host__ __device__ void for_k(int nv, F fn)
@@ -43,7 +46,7 @@ struct GX {
 #endif
     }
 
-    // Deterministic workgroup sum of v[N], result in every lane: butterfly within each wavefront,
+    // Deterministic workgroup sum of v[N], result in every lane: over the lanes of each wavefront,
     // then the wavefront totals added in order.
     template <int N>
     __host__ __device__ void sum(double *v)
@@ -51,17 +54,10 @@ struct GX {
         static_assert(N <= SUM_MAX, "reduction width");
 #if defined(__HIP_DEVICE_COMPILE__)
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            double x = v[i];
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-            v[i] = x;
-        }
+        lane_sums<N>(v, lane);
+        const int q = lane_value<N>(lane, 0);
         __syncthreads();
-        if (lane == 0)
-#pragma unroll
-            for (int i = 0; i < N; ++i) lds[wave * N + i] = v[i];
+        if (q >= 0) lds[wave * N + q] = v[0];
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < N; ++i) {
@@ -85,16 +81,25 @@ struct GX {
     }
 };
 
-template <class Tag, class Fn>
-__global__ __launch_bounds__(NT) void k_points(Fn fn)
+// k_face_adj takes 146 registers left alone, 3 waves a SIMD: 323 us for 16000 faces of 32^2 velocities,
+// 294 with 4 waves.  The others fit, or spill inside their loops when held to more.
+template <class Tag>
+constexpr int min_waves()
+{
+    return std::is_same_v<Tag, adj::k_face_adj> ? 4 : 1;
+}
+
+template <class Tag, int NT, bool ROWS, class Fn>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(min_waves<Tag>(), 8))) void k_points(Fn fn)
 {
     __shared__ double lds[(NT / 64) * SUM_MAX];
-    GX x{lds};
+    extern __shared__ __align__(16) double rows[];
+    GX<NT, ROWS> x{lds, rows};
     fn(x, (int)blockIdx.x);
 }
 
 struct HipBackend {
-    int device = 0;
+    int device = 0, nv = 0;   // nv: velocities of a point
     hipStream_t stream = nullptr;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     bool bad = false;
@@ -173,11 +178,31 @@ struct HipBackend {
         if (bytes) check(hipMemsetAsync(d, 0, bytes, stream), "memset");
     }
 
+    template <class Tag, int NT, class Fn>
+    void launch_nt(int n, Fn fn)
+    {
+        const size_t rows = 2 * (size_t)nv * sizeof(double);
+        if constexpr (adj::uses_rows<Tag>::value) {
+            if (rows <= ROWS_MAX) {
+                hipLaunchKernelGGL((k_points<Tag, NT, true, Fn>), dim3(n), dim3(NT), rows, stream, fn);
+                return;
+            }
+        }
+        hipLaunchKernelGGL((k_points<Tag, NT, false, Fn>), dim3(n), dim3(NT), 0, stream, fn);
+    }
+
     template <class Tag, class Fn>
     void launch(int n, Fn fn)
     {
         if (n <= 0 || bad) return;
-        hipLaunchKernelGGL((k_points<Tag, Fn>), dim3(n), dim3(NT), 0, stream, fn);
+        // Lanes of a point: 64 up to 128 velocities (50^2 cells of 9^2: 8.5 ms for 60 steps, 9.2 with 128), 128
+        // beyond (200 x 40 cells of 32^2: 128 ms, 166 with 64), and more while the points give the
+        // device fewer than NT_FILL waves (20^2 cells of 28^2: 14.2 ms with 128, 11.3 with 256)
+        int nt = nv <= 128 ? 64 : 128;
+        while (nt < 256 && nt < nv && (long)n * (nt / 64) < NT_FILL) nt *= 2;
+        if (nt == 64) launch_nt<Tag, 64>(n, fn);
+        else if (nt == 128) launch_nt<Tag, 128>(n, fn);
+        else launch_nt<Tag, 256>(n, fn);
         check(hipGetLastError(), "kernel launch");
     }
 
@@ -224,6 +249,7 @@ int dugks_adjoint_create(const dugks_case *cs, dugks_adjoint **out)
         a->e.err = "no usable HIP device: " + a->e.be.msg;
     } else {
         rc = a->e.create(cs);
+        a->e.be.nv = a->e.p.nv;
     }
     *out = a;   // returned also on failure so that dugks_adjoint_last_error can explain it
     return rc;
