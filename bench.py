@@ -40,6 +40,8 @@ def bytes_model(case, storage_bytes: int, n_blocks: int, n_blocks_cell: int = No
     k_cell_s1 reads g~ and writes the next gbar; the two _fin kernels touch O(faces) and
     O(cells) data.  With fused_cell, k_cell also forms the macros and the next gbar in place
     (k_cell_fin and k_cell_s1 do not run; the re-read of its own row adds nothing to the floor).
+    The column kernels are timed in the same slots: their face pass (k_face_lines, in k_face_values)
+    forms the moments itself and leaves the k_face_moments slot empty; k_cell_lines is k_cell.
     h is carried only when K + 3 - D != 0.  The whole-step figure is the
     floor of the scheme: gbar read twice and written once (3 s per update), plus the face
     values written and read once in face-value mode."""

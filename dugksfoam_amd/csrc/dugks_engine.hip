@@ -2446,7 +2446,7 @@ void shape_candidates(dugks_engine *h)
 //     160 and 140 us with 1, 2 and 3 waves a cell, 1, 2 and 2 rounds); past a few rounds the last one's
 //     idle half is what counts.
 // At most 4 waves a cell: 48^3 cells of 24^3 velocities take 34.4 ms with 3, 49.7 with 5.
-constexpr double TILE_COST = 0.8, MIX_COST = 0.2, WAVE_COST = 2.0;
+constexpr double TILE_COST = 0.8, MIX_COST = 0.1, WAVE_COST = 2.0;
 
 void velocity_columns(int D, int nxi, const double *xi, int nc, int slots, int line, std::vector<LineRec> &recs,
                       std::vector<int> &titer, std::vector<int> &slot_ref, int &waves)
@@ -3274,6 +3274,7 @@ int step_impl(dugks_engine *h, const double *dtc, int nsteps)
         for (int s = 0; s < nsteps; ++s) {
             const hipEvent_t *e = &h->pev[(NKERN + 1) * (size_t)s];
             for (int i = 0; i < NKERN; ++i) {
+                if (i == 1 && use_lines(h)) continue;   // no second face pass: two events in a row
                 float a = 0.f;
                 HIPCHK(h, hipEventElapsedTime(&a, e[i], e[i + 1]));
                 h->prof[i] += a;
