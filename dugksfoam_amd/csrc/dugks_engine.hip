@@ -46,6 +46,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <limits>
 #include <mutex>
 #include <new>
 #include <numeric>
@@ -69,6 +70,7 @@ constexpr int KIND_FAR = 5;   // incoming Maxwellian: far field (farField rho) o
 constexpr int KIND_ZG = 6;    // zeroGradient: every face value is the owner cell's gBarPvol
 constexpr int KIND_SPL = 7;   // OpenFOAM symmetryPlane: mirror plane, gBarPvol phi_b = phi_P (no lagged
                               // row), every value relaxed by the field operation, outgoing ones twice
+constexpr int KIND_NONE = -1;  // column kernels: a slot past the cell's faces
 
 // Boundary faces with a lagged fixedGradient gBarPvol row; open faces relax only outgoing values.
 __host__ __device__ constexpr inline bool grad_row(int kind)
@@ -208,8 +210,9 @@ struct alignas(64) LineFace {
 };
 
 // Geometry of a (cell, face) slot for the column kernels: centre to face, and the outward area
-// vector, its loop-axis component apart.  NS entries per cell; those past its faces have S = 0 and
-// the cell's first face.
+// vector, its loop-axis component apart.  NS entries per cell.  Those past its faces (KIND_NONE) name the
+// cell's first face, whose row is loaded and dropped; their Sl is a NaN, so that xi.S compares false
+// with everything: no velocity is upwind of them, and none runs along them.
 struct alignas(64) LineGeo {
     double dC[3];
     double S[2], Sl, pad;
@@ -2910,7 +2913,8 @@ int build(dugks_engine *h, const dugks_case *cs)
             LineGeo &g = lgeo[(size_t)c * lns + j];
             std::memset(&g, 0, sizeof g);
             g.face = sl[cnt[c]].face;
-            g.kind = KIND_OWN;
+            g.kind = KIND_NONE;
+            g.Sl = std::numeric_limits<double>::quiet_NaN();
             if (cnt[c] + j >= cnt[c + 1]) continue;
             const Slot &q = sl[cnt[c] + j];
             const double sgn = q.kind == KIND_NEI ? -1.0 : 1.0;

@@ -389,7 +389,7 @@ __global__ __launch_bounds__(LINE_MAXNT) __attribute__((amdgpu_waves_per_eu(D ==
             if (D == 2) return col.x * Sx[j] + l;
             return (col.x * Sx[j] + col.y * Sy[j]) + l;
         };
-        // velocities along a face: |xi.S| < VSMALL (also the padding entries, S = 0)
+        // velocities along a face: |xi.S| < VSMALL (none of a slot past the cell's faces: xi.S is a NaN)
         bool mid = false;
 #pragma unroll
         for (int j = 0; j < NS; ++j) mid = mid || fabs(flux_dir(j)) < VSMALL;
@@ -448,7 +448,7 @@ __global__ __launch_bounds__(LINE_MAXNT) __attribute__((amdgpu_waves_per_eu(D ==
                 if (H) hf = fma(HC[d], dc, hf);
             }
             const int kind = BND || anymid ? LG[j].kind : KIND_OWN;
-            // the values this cell writes: where it is upwind (outward xi.S)
+            // the values this cell writes: where it is upwind (outward xi.S; never on KIND_NONE)
             bool mine = s > 0.0, own = true;
             double part = 1.0;
             if (anymid && (kind == KIND_OWN || kind == KIND_NEI)) {

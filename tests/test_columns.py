@@ -11,6 +11,7 @@ import dataclasses
 import numpy as np
 import pytest
 
+import mixed_meshes as mm
 from dugksfoam_amd import cases
 from dugksfoam_amd.engine import Engine
 
@@ -91,4 +92,108 @@ def test_columns_match_the_oracle(which, oracle_lib, monkeypatch):
         assert _off(c, e.macro(), r.macro()) <= tol
         e.close()
         r.close()
+    o.close()
+
+
+def _on_columns(e):
+    """True when the engine runs the column kernels: they have one shape, and nothing is tuned."""
+    e.autotune(True)
+    left = e.autotune_steps_left()
+    e.autotune(False)
+    return left == 0
+
+
+def _box(dim, cells, name, nv, K=0, **sides):
+    """The unit square or cube of the given cells; walls, the y1 one moving, but for `sides`."""
+    p = {a + s: mm.wall(20.0 if a + s == "y1" else 0.0) for a in "xyz"[:dim] for s in "01"}
+    p.update(sides)
+    return mm.build(name, *cells, mm.box_side(dim), p, dim, nv, K=K)
+
+
+def _islands_2d(K, first):
+    """Triangles beside two quads, each cell on its own.  The first two triangles couple their vertical edges
+    (a cyclic pair); the first face of the third is a far field; the fourth has walls only."""
+    pts, cells = [], []
+    shapes = [[(0, 0), (1, 0), (0, 1)], [(5, 0), (5, 1), (4, 1)], [(6, 0), (7, 0), (6, 1)], [(8, 0), (9, 0), (9, 1)],
+              [(10, 0), (11, 0), (11, 1), (10, 1)], [(11, 0), (12, 0), (12, 1), (11, 1)]]
+    for s in shapes:
+        n = len(pts)
+        pts += [(x, y, z) for z in (0.0, 0.1) for x, y in s]
+        k = len(s)
+        cells.append(mm._prism(list(range(n, n + k)), list(range(n + k, n + 2 * k))))
+
+    def patch(x, n):
+        if abs(n[2]) > 0.9:
+            return None
+        if abs(n[0]) > 0.999 and x[0] in (0.0, 5.0):
+            return "c0" if x[0] == 0.0 else "c1"
+        return "far" if abs(x[0] - 6.0) < 1e-9 else "walls"
+
+    kinds = {"c0": mm.cyclic(1), "c1": mm.cyclic(0), "far": first, "walls": mm.wall(15.0)}
+    return mm.build("islands", pts, cells, patch, kinds, 2, 13, K=K)
+
+
+def _islands_3d(K):
+    """Single prisms and tetrahedra: two prisms coupled by a cyclic pair, a tetrahedron with a far field first,
+    one with walls only."""
+    pts, cells = [], []
+    for s in ([(0, 0), (1, 0), (0, 1)], [(5, 0), (5, 1), (4, 1)]):
+        n = len(pts)
+        pts += [(x, y, z) for z in (0.0, 1.0) for x, y in s]
+        cells.append(mm._prism([n, n + 1, n + 2], [n + 3, n + 4, n + 5]))
+    for x in (6.0, 8.0):
+        n = len(pts)
+        pts += [(x, 0, 0), (x + 1, 0, 0), (x, 1, 0), (x, 0, 1)]
+        cells.append([[n + i for i in range(4) if i != j] for j in range(4)])
+
+    def patch(x, n):
+        if abs(n[0]) > 0.999 and x[0] in (0.0, 5.0):
+            return "c0" if x[0] == 0.0 else "c1"
+        return "far" if abs(x[0] - 6.0) < 1e-9 else "walls"
+
+    kinds = {"c0": mm.cyclic(1), "c1": mm.cyclic(0), "far": mm.far_field, "walls": mm.wall(15.0)}
+    return mm.build("islands3d", pts, cells, patch, kinds, 3, 7, K=K)
+
+
+def _strip(nz=1):
+    """Quads (hexahedra) in one row between walls, every third column cut into two triangles (prisms): each
+    cell has a wall."""
+    return mm.split_columns(7, 1, nz, lambda i, j: i % 3 != 1)
+
+
+# Cells with fewer faces than the kernels have slots, each with a wall or an open face
+PADDED = {
+    "strip": lambda: _box(2, _strip(), "strip", 12),
+    "strip_odd_K2": lambda: _box(2, _strip(), "strip", 9, K=2),
+    "strip_cyclic": lambda: _box(2, _strip(), "strip", 13, x0=mm.cyclic(1), x1=mm.cyclic(0)),
+    "strip_pressure": lambda: _box(2, _strip(), "strip", 11, K=2, x0=mm.pressure_in, x1=mm.far_field),
+    "strip_zero_gradient": lambda: _box(2, _strip(), "strip", 10, x0=mm.far_field, x1=mm.zero_gradient),
+    "strip_mirror": lambda: _box(2, _strip(), "strip", 11, y0=mm.mirror("symmetryMod")),
+    "strip_plane": lambda: _box(2, _strip(), "strip", 8, y0=mm.mirror("symmetryPlane")),
+    "islands": lambda: _islands_2d(0, mm.far_field),
+    "islands_K2": lambda: _islands_2d(2, mm.pressure_in),
+    "prisms": lambda: _box(3, _strip(3), "prisms", 7),
+    "prisms_K2": lambda: _box(3, _strip(2), "prisms", 6, K=2, x0=mm.cyclic(1), x1=mm.cyclic(0)),
+    "pyramids": lambda: _box(3, mm.split_pyramids(1, lambda i, j, k: True), "pyramids", 9, z1=mm.far_field),
+    "pyramids_K2": lambda: _box(3, mm.split_pyramids(1, lambda i, j, k: True), "pyramids", 6, K=2),
+    "islands_3d": lambda: _islands_3d(0),
+    "islands_3d_K2": lambda: _islands_3d(2),
+}
+
+
+@pytest.mark.parametrize("which", list(PADDED))
+def test_cells_with_fewer_faces_than_slots(which, oracle_lib):
+    c = PADDED[which]()
+    o = oracle_lib.Oracle(c)
+    o.init_equilibrium()
+    o.step(nsteps=4)
+    for storage, tol in (("fp64", 1e-12), ("fp32", 1e-6)):
+        print(which, storage, flush=True)
+        e = Engine(c, storage=storage)
+        assert _on_columns(e)
+        e.init_equilibrium()
+        e.step(nsteps=4)
+        assert _off(c, e.macro(), o.macro()) <= tol
+        assert _off(c, e.face_macro(), o.face_macro()) <= tol
+        e.close()
     o.close()
