@@ -204,7 +204,8 @@ struct LineRec;   // lines.h
 struct LineCell;  // lines.h
 
 // What the column form of k_cell needs of a (cell, face) slot in every iteration: the face
-// equilibrium along the loop axis, 1 - r, and +-S dt / V of that axis.  Written by k_face_fin.
+// equilibrium along the loop axis, 1 - r, and +-S dt / V of that axis.  Written by k_face_fin; 0 in the
+// slots past a cell's faces.
 struct alignas(64) LineFace {
     double invRT, B, qz, omr, Sl, RT, pad[2];
 };
@@ -3058,6 +3059,9 @@ int build(dugks_engine *h, const dugks_case *cs)
          (r = dalloc(h, &h->opart, open_faces.size() * NMom<3>::v)) || (r = dalloc(h, &h->lface, (size_t)nc * lns)) || (r = dalloc(h, &h->lcell, (size_t)nc)) ||
          (r = dalloc(h, &h->fslot, nf)) || (r = upload(h, h->fslot, fslot.data(), nf))))
         return r;
+    // k_face_fin writes the slots of the cells' faces; the others stay 0, so that the loops of
+    // k_cell_lines over all slots add nothing there
+    if (h->line_ok) HIPCHK(h, hipMemsetAsync(h->lface, 0, sizeof(LineFace) * (size_t)nc * lns, h->stream));
     if (nw && (r = upload(h, h->wall, wc.data(), nw))) return r;
     if (nw && ((r = dalloc(h, &h->bpress, nw)) || (r = upload(h, h->bpress, wpress.data(), nw)))) return r;
     h->nopen = (int)open_faces.size();
