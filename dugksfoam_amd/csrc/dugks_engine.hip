@@ -2136,6 +2136,16 @@ void launch_step_fv(dugks_engine *h, hipEvent_t *ev)
 // Column kernels run in face-value mode with the default face moments.
 bool use_lines(const dugks_engine *h) { return h->line_ok && h->face_values && h->face_mfma && !h->face_pass_legacy; }
 
+// Slots per cell of the column kernels on a mesh of cells of up to ns_max faces.  They work on every
+// slot, so meshes of triangles and of tetrahedra have their own: 8640 tetrahedra, 12^3 velocities, 6 slots and
+// 4: 548 and 441 us FP64, 503 and 411 FP32 (k_face_values and k_cell: 501 and 420).  Meshes that mix cells keep
+// the larger count: 60^2 quads, a third of them two triangles, 28^2 velocities: 180 us FP64, 154 FP32
+// (k_face_values and k_cell: 194, 168).
+int line_slots(int D, int ns_max)
+{
+    return D == 1 ? 2 : (D == 2 ? (ns_max <= 3 ? 3 : 4) : (ns_max <= 4 ? 4 : 6));
+}
+
 // LDS bytes of the column kernels (k_cell_lines: without the new row)
 template <int D, bool H, int NS>
 size_t line_face_lds(const dugks_engine *h, int waves)
@@ -2208,9 +2218,12 @@ void launch_step_ns(dugks_engine *h, hipEvent_t *ev)
         if (use_lines(h)) {
             if constexpr (D == 1) return launch_step_lines<D, H, 2, TS>(h, ev);
             else if constexpr (D == 2) {
-                if (h->ns_max <= 3) return launch_step_lines<D, H, 3, TS>(h, ev);
+                if (line_slots(D, h->ns_max) == 3) return launch_step_lines<D, H, 3, TS>(h, ev);
                 return launch_step_lines<D, H, 4, TS>(h, ev);
-            } else return launch_step_lines<D, H, NS, TS>(h, ev);
+            } else {
+                if (line_slots(D, h->ns_max) == 4) return launch_step_lines<D, H, 4, TS>(h, ev);
+                return launch_step_lines<D, H, NS, TS>(h, ev);
+            }
         }
     }
     if (h->face_values) launch_step_fv<D, H, NS, TS, true>(h, ev);
@@ -2906,7 +2919,7 @@ int build(dugks_engine *h, const dugks_case *cs)
             }
         for (int k = 0; k < nv; ++k) img_slot[k] = slot[order[k]];
     }
-    const int lns = D == 1 ? 2 : (D == 2 ? (h->ns_max <= 3 ? 3 : 4) : 6);   // slots per cell of the column kernels
+    const int lns = line_slots(D, h->ns_max);
     std::vector<int4> fslot(nf, int4{-1, -1, -1, 0});
     std::vector<LineGeo> lgeo(h->line_ok ? (size_t)nc * lns : 0);
     for (int c = 0; c < nc && h->line_ok; ++c)
