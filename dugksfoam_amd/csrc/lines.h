@@ -39,6 +39,10 @@ constexpr int line_nval()
 constexpr int LINE_MAXW = 8;             // waves per workgroup
 constexpr int LINE_MAXNT = 64 * LINE_MAXW;
 
+// LDS by its own address space, where one value comes from LDS or from memory: through generic pointers the
+// compiler merges the two loads into one flat load behind a null check.
+#define LDS_AS __attribute__((address_space(3)))
+
 template <typename T>
 DEVI T ld_at(const T *base, unsigned byte_off)
 {
@@ -679,7 +683,7 @@ DEVI void line_s1(const P<TS> &p, int c, const CellEq &e, const double *tabC, co
     const double mog = vt[3 * p.nax], moh = vt[3 * p.nax + 1], kc2K = 2.0 * p.kc - 2.0 * p.K;
     double g0, P0, q0;
     bool inL = false;
-    TS *rl = rowL;
+    LDS_AS TS *const rL = (LDS_AS TS *)rowL, *rl = rL;
     struct None {};
     walk_columns<D, LT, None>(
         p, vt, tab,
@@ -688,7 +692,7 @@ DEVI void line_s1(const P<TS> &p, int c, const CellEq &e, const double *tabC, co
             line_fixed<D>(e, col.x, col.y, P0, q0);
             if (LDS) {
                 inL = t < p.ntl;
-                rl = rowL + (inL ? __builtin_amdgcn_readfirstlane(p.titer[t]) : 0) * (H ? 128 : 64) + (threadIdx.x & 63);
+                rl = rL + (inL ? __builtin_amdgcn_readfirstlane(p.titer[t]) : 0) * (H ? 128 : 64) + (threadIdx.x & 63);
             }
         },
         [](unsigned, None &) {},
@@ -819,7 +823,7 @@ __global__ __launch_bounds__(LINE_MAXNT) __attribute__((amdgpu_waves_per_eu(D ==
         if (H) pin(cRT);
     }
     bool inL = false;
-    TS *rl = rowL;
+    LDS_AS TS *const rL = (LDS_AS TS *)rowL, *rl = rL;
 
     struct Rows {
         TS g, h, fg[NS], fh[H ? NS : 1];
@@ -843,7 +847,7 @@ __global__ __launch_bounds__(LINE_MAXNT) __attribute__((amdgpu_waves_per_eu(D ==
             for (int m = 0; m < NA; ++m) n[m] = 0.0;
             if (F1) {
                 inL = t < p.ntl;
-                rl = rowL + (inL ? __builtin_amdgcn_readfirstlane(p.titer[t]) : 0) * (H ? 128 : 64) + lane;
+                rl = rL + (inL ? __builtin_amdgcn_readfirstlane(p.titer[t]) : 0) * (H ? 128 : 64) + lane;
             }
         },
         [&](unsigned ko, Rows &r) {
@@ -897,7 +901,7 @@ __global__ __launch_bounds__(LINE_MAXNT) __attribute__((amdgpu_waves_per_eu(D ==
                     // field operation, 880-881), the outgoing ones once more (905-920)
                     const bool all = kind == KIND_OWN || kind == KIND_NEI || kind == KIND_CYC || kind == KIND_SPL;
                     if (kind == KIND_WALL && !(so > 0)) {
-                        const int l = (int)(e - tab) / LT;
+                        const int l = (int)((LDS_AS const double *)e - (LDS_AS const double *)tab) / LT;
                         g = tabW[(la0 + l) * NS + j];
                         if (D >= 2) g *= tabW[col.ix * NS + j];
                         if (D == 3) g *= tabW[(nxi + col.iy) * NS + j];
