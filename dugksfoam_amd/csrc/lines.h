@@ -586,10 +586,10 @@ struct CellEq {
     double invRT, RT, pre, B[3], C0, Q0, qc[3];
 };
 
-// What the column form of k_cell needs of the state that formed gbar: the cell equilibrium and the
-// factors of -1/3 g~ + 4/3 gbar = cA gbar + cB geq.  Written by k_face_fin.
+// What the column form of k_cell needs of the state that formed gbar: the cell equilibrium and
+// kr = r / (1 - r) of g~ (s8_cell).  Written by k_face_fin.
 struct alignas(64) LineCell {
-    double invRT, B[3], qc[3], RT, cA, cB, pre, C0, Q0, dtV, pad[2];
+    double invRT, B[3], qc[3], RT, kr, pre, C0, Q0, dtV, pad[3];
 };
 static_assert(sizeof(LineCell) == 128, "linecell size");
 
@@ -613,13 +613,22 @@ DEVI void cell_eq(double rho, const double *U, double T, const double *q, double
     e.Q0 = -uq;
 }
 
+// -1/3 g~ + 4/3 gbar with g~ = (gbar - r geq) / (1 - r) = gbar - kr (geq - gbar).  In this form the rounding
+// of kr takes nothing from the cell's sums, which geq - gbar does not hold: with cA gbar + cB geq, cA + cB is
+// 1 within the last place of cA only, a loss of mass in every step that grows without bound as r nears 1.
+DEVI double s8_cell(double g, double geq, double kr)
+{
+    const double gt = fma(-kr, geq - g, g);
+    return fma(4.0 / 3, g, -1.0 / 3 * gt);
+}
+
 template <int D, typename TS>
 DEVI void line_cell(const P<TS> &p, int c)
 {
     const double dt = p.dtc[p.ccase[c]];
     CellEq e;
     cell_eq<D>(p.crho[c], p.cU + 3 * (size_t)c, p.cT[c], p.cq + 3 * (size_t)c, p.R, p.Pr, e);
-    const double r = s1_r(dt, p.ctau[c]), inv1mr = 1.0 / (1.0 - r);
+    const double r = s1_r(dt, p.ctau[c]);
     LineCell lc;
     lc.invRT = e.invRT;
     lc.RT = e.RT;
@@ -630,10 +639,9 @@ DEVI void line_cell(const P<TS> &p, int c)
         lc.B[d] = e.B[d];
         lc.qc[d] = e.qc[d];
     }
-    lc.cA = 4.0 / 3 - inv1mr / 3;
-    lc.cB = r * inv1mr / 3;
+    lc.kr = r / (1.0 - r);
     lc.dtV = dt / p.cV[c];
-    lc.pad[0] = lc.pad[1] = 0.0;
+    lc.pad[0] = lc.pad[1] = lc.pad[2] = 0.0;
     p.lcell[c] = lc;
 }
 
@@ -813,10 +821,9 @@ __global__ __launch_bounds__(LINE_MAXNT) __attribute__((amdgpu_waves_per_eu(D ==
         pin(LF[j].Sl);
         if (H) pin(LF[j].RT);
     }
-    double cA = LC->cA, cB = LC->cB, cinvRT = LC->invRT, cBl = LC->B[D - 1], cqz = LC->qc[D - 1], cRT = H ? LC->RT : 0.0;
+    double kr = LC->kr, cinvRT = LC->invRT, cBl = LC->B[D - 1], cqz = LC->qc[D - 1], cRT = H ? LC->RT : 0.0;
     if (VEC) {
-        pin(cA);
-        pin(cB);
+        pin(kr);
         pin(cinvRT);
         pin(cBl);
         pin(cqz);
@@ -870,8 +877,8 @@ __global__ __launch_bounds__(LINE_MAXNT) __attribute__((amdgpu_waves_per_eu(D ==
             double geq, heq;
             line_geq<H>(z, cinvRT, cBl, cqz, cRT, cP0, cq0, c0 * e[6], p.kc, kc2K, geq, heq);
             // S8 (discreteVelocity.C:937-975): -1/3 g~ + 4/3 gbar with g~ = (gbar - r geq) / (1 - r)
-            double ag = fma(cA, gC, cB * geq);
-            double ah = H ? fma(cA, hC, cB * heq) : 0.0;
+            double ag = s8_cell(gC, geq, kr);
+            double ah = H ? s8_cell(hC, heq, kr) : 0.0;
             if (plain) {
 #pragma unroll
                 for (int j = 0; j < NS; ++j) {
