@@ -2464,7 +2464,7 @@ void shape_candidates(dugks_engine *h)
 //     idle half is what counts.
 // At most 4 waves a cell: 48^3 cells of 24^3 velocities take 34.4 ms with 3, 49.7 with 5.
 constexpr double TILE_COST = 0.8, MIX_COST = 0.1, WAVE_COST = 2.0;
-
+// The columns are built once, for the m chosen; the search goes over runs of columns of one length and class.
 void velocity_columns(int D, int nxi, const double *xi, int nc, int slots, int line, std::vector<LineRec> &recs,
                       std::vector<int> &titer, std::vector<int> &slot_ref, int &waves)
 {
@@ -2480,15 +2480,11 @@ void velocity_columns(int D, int nxi, const double *xi, int nc, int slots, int l
                 if (v[i].n > s) r.push_back({v[i].ix, v[i].iy, v[i].l + s * v[i].dl, v[i].dl * m, (v[i].n - s + m - 1) / m});
         return r;
     };
-    std::vector<Col> best;
-    double best_cost = -1.0;
-    for (int m = 1; m <= nxi; ++m) {
-        // 2-D: at least 24 lanes of one sign class together where there are as many: 14-lane runs (28 points,
-        // m = 1) take the batch's face pass 3.1 ms, 28-lane runs 2.3 ms (partly written cache lines)
-        if (D == 2 && m * (int)ax[2].size() < 24 && m < nxi) continue;
+    const int ncy = D == 3 ? 3 : 1, ncx = D >= 2 ? 3 : 1;
+    auto columns = [&](int m) {
         std::vector<Col> v;
-        for (int cy = 0; cy < (D == 3 ? 3 : 1); ++cy)
-            for (int cx = 0; cx < (D >= 2 ? 3 : 1); ++cx) {
+        for (int cy = 0; cy < ncy; ++cy)
+            for (int cx = 0; cx < ncx; ++cx) {
                 std::vector<Col> q;
                 for (int y = 0; y < (D == 3 ? (int)ax[cy].size() : 1); ++y)
                     for (int x = 0; x < (D >= 2 ? (int)ax[cx].size() : 1); ++x)
@@ -2503,31 +2499,88 @@ void velocity_columns(int D, int nxi, const double *xi, int nc, int slots, int l
             v.resize(full);
             v.insert(v.end(), q.begin(), q.end());
         }
-        std::vector<double> tile;
-        for (size_t i = 0; i < v.size(); i += 64) {
-            const size_t i1 = std::min(v.size(), i + 64);
-            int its = 0;
-            bool mix = false;
-            for (size_t k = i; k < i1; ++k) {
-                its = std::max(its, v[k].n);
-                mix = mix || (D == 2 && k % line && sgn(xi[v[k].ix]) != sgn(xi[v[k - 1].ix]));
+        return v;
+    };
+    // the tiles' costs of columns(m), from its runs {length, columns, class}
+    struct Run { int n, cnt, cls; };
+    std::vector<Run> runs;
+    std::vector<double> tile;
+    auto tile_costs = [&](int m) {
+        runs.clear();
+        tile.clear();
+        int total = 0;
+        for (int cy = 0; cy < ncy; ++cy)
+            for (int cx = 0; cx < ncx; ++cx) {
+                const int cnt = (D == 3 ? (int)ax[cy].size() : 1) * (D >= 2 ? (int)ax[cx].size() : 1);
+                for (int s = 0; s < m && cnt; ++s) runs.push_back({(nxi - s + m - 1) / m, cnt, cx});
+                total += m * cnt;
             }
-            tile.push_back(its * (mix ? 1 + MIX_COST : 1) + TILE_COST);
+        size_t r = 0;
+        int used = 0, its = 0, cls = -1;   // columns taken of run r; the tile's longest column, its last class
+        bool mix = false;
+        auto put = [&] { tile.push_back(its * (mix ? 1 + MIX_COST : 1) + TILE_COST); };
+        for (int i = 0; i + 64 <= total; i += 64) {
+            its = 0;
+            mix = false;
+            for (int lane = 0; lane < 64;) {
+                if (used == runs[r].cnt) {
+                    ++r;
+                    used = 0;
+                }
+                its = std::max(its, runs[r].n);
+                mix = mix || (D == 2 && lane % line && runs[r].cls != cls);
+                cls = runs[r].cls;
+                const int c = std::min(64 - lane, runs[r].cnt - used);
+                used += c;
+                lane += c;
+            }
+            put();
         }
+        if (const int left = total % 64) {
+            int n[64], c[64];
+            for (int i = left, q = (int)runs.size() - 1, u = 0; i--;) {
+                n[i] = runs[q].n;
+                c[i] = runs[q].cls;
+                if (++u == runs[q].cnt) {
+                    --q;
+                    u = 0;
+                }
+            }
+            const int k = std::min(64 / left, n[0]);
+            its = (*std::max_element(n, n + left) + k - 1) / k;
+            mix = false;
+            for (int part = 0, lane = 0; part < k; ++part)
+                for (int i = 0; i < left; ++i) {
+                    if (n[i] <= part) continue;
+                    mix = mix || (D == 2 && lane % line && c[i] != cls);
+                    cls = c[i];
+                    ++lane;
+                }
+            put();
+        }
+    };
+    int best_m = 1;
+    double best_cost = -1.0;
+    for (int m = 1; m <= nxi; ++m) {
+        // 2-D: at least 24 lanes of one sign class together where there are as many: 14-lane runs (28 points,
+        // m = 1) take the batch's face pass 3.1 ms, 28-lane runs 2.3 ms (partly written cache lines)
+        if (D == 2 && m * (int)ax[2].size() < 24 && m < nxi) continue;
+        tile_costs(m);
         for (int w = 1; w <= std::min(4, (int)tile.size()); ++w) {
-            std::vector<double> busy(w, WAVE_COST);
+            double busy[4] = {WAVE_COST, WAVE_COST, WAVE_COST, WAVE_COST};
             for (size_t t = 0; t < tile.size(); ++t) busy[t % w] += tile[t];
-            const double b = *std::max_element(busy.begin(), busy.end());
+            const double b = *std::max_element(busy, busy + w);
             const double x = (double)nc * w / slots, rounds = x < 3 ? std::ceil(x) : x + 0.5;
             const double lone = 0.35 * std::min(1.0, std::max(0.0, (b - 20) / 13)), tail = 0.1 * std::max(0.0, std::log2(b / 13));
             const double cost = rounds * b * (1 + (x <= 1 ? lone : tail));
             if (best_cost < 0 || cost < best_cost) {
-                best = v;
+                best_m = m;
                 best_cost = cost;
                 waves = w;
             }
         }
     }
+    const std::vector<Col> best = columns(best_m);
     titer.assign(1, 0);
     for (size_t i0 = 0; i0 < best.size(); i0 += 64) {
         const int q0 = titer.back();
@@ -3057,12 +3110,6 @@ int build(dugks_engine *h, const dugks_case *cs)
         (r = upload(h, h->fx, fxs.data(), nf)) || (r = upload(h, h->cst, cst.data(), nc)) ||
         (r = upload(h, h->corder, corder.data(), nc)) || (r = upload(h, h->forder, forder.data(), nf)) || (r = upload(h, h->wfslot, wfslot.data(), nw)))
         return r;
-    // rows are padded to nvp; the column kernels write the nv velocities only, the others read the
-    // padding with weight 0
-    for (int i = 0; i < 2; ++i) {
-        HIPCHK(h, hipMemset(h->gb[i], 0, row + brow));
-        if (h->has_h) HIPCHK(h, hipMemset(h->hb[i], 0, row + brow));
-    }
     if (h->line_ok &&
         ((r = dalloc(h, &h->img_slot, img_slot.size())) || (r = upload(h, h->img_slot, img_slot.data(), img_slot.size())) ||
          (r = dalloc(h, &h->rec, recs.size())) || (r = upload(h, h->rec, recs.data(), recs.size())) ||
@@ -3326,6 +3373,17 @@ void image_rows(dugks_engine *h, void *img, void *rows, int save)
         hipLaunchKernelGGL((k_image<float>), dim3(n), dim3(256), 0, h->stream, (float *)img, (float *)rows, h->img_slot, h->nvp_img, h->nvp, save);
     else
         hipLaunchKernelGGL((k_image<double>), dim3(n), dim3(256), 0, h->stream, (double *)img, (double *)rows, h->img_slot, h->nvp_img, h->nvp, save);
+}
+
+// Zeros a ping-pong side that staged an image.  The column kernels write the nv velocities of a row only; what
+// reads the padding gives it weight 0, so it has to be finite (dugks_init_equilibrium and the conversion
+// that follows write all of a row).
+int clear_side(dugks_engine *h, int side)
+{
+    const size_t bytes = ((size_t)h->nc + (h->nw ? h->nw : 1)) * h->nvp * ts_size(h);
+    HIPCHK(h, hipMemsetAsync(h->gb[side], 0, bytes, h->stream));
+    if (h->has_h) HIPCHK(h, hipMemsetAsync(h->hb[side], 0, bytes, h->stream));
+    return 0;
 }
 
 const int64_t STATE_MAGIC = 0x44554b5331LL;  // "DUKS1"
@@ -3705,6 +3763,8 @@ int dugks_save_state(dugks_engine *h, void *buf, int64_t bytes)
     if (h->has_h) { HIPCHK(h, hipMemcpy(p, hr, row, hipMemcpyDeviceToHost)); p += row; }
     HIPCHK(h, hipMemcpy(p, gr + row, brow, hipMemcpyDeviceToHost)); p += brow;
     if (h->has_h) { HIPCHK(h, hipMemcpy(p, hr + row, brow, hipMemcpyDeviceToHost)); p += brow; }
+    if (h->line_ok)
+        if (int rr = clear_side(h, side)) return rr;
     const size_t nc = h->nc;
     HIPCHK(h, hipMemcpy(p, h->crho, 8 * nc, hipMemcpyDeviceToHost)); p += 8 * nc;
     HIPCHK(h, hipMemcpy(p, h->cU, 24 * nc, hipMemcpyDeviceToHost)); p += 24 * nc;
@@ -3746,6 +3806,7 @@ int dugks_load_state(dugks_engine *h, const void *buf, int64_t bytes)
         image_rows(h, gr, h->gb[h->cur], 0);
         if (h->has_h) image_rows(h, hr, h->hb[h->cur], 0);
         HIPCHK(h, hipGetLastError());
+        if (int rr = clear_side(h, side)) return rr;
         HIPCHK(h, hipStreamSynchronize(h->stream));
     }
     const size_t nc = h->nc;
