@@ -3265,7 +3265,7 @@ int step_impl(dugks_engine *h, const double *dtc, int nsteps)
     // online launch-shape tuning: each step runs the next candidate shape of k_face and of
     // k_cell (after one warm-up step), timed with events; every candidate is timed in
     // TUNE_ROUNDS rounds and the one with the shortest time of each kernel is kept
-    while (h->tuning && s0 < nsteps) {
+    while (h->tuning && !use_lines(h) && s0 < nsteps) {
         const int nfc = (int)h->face_cand.size(), ncc = (int)h->cell_cand.size();
         const int ncand = std::max(nfc, ncc);
         const int i = h->tune_i < 0 ? -1 : h->tune_i % ncand;
@@ -3837,7 +3837,7 @@ int dugks_last_step_ms(dugks_engine *h, double *ms)
 int dugks_set_autotune(dugks_engine *h, int32_t on)
 {
     if (!h) return DUGKS_ERR_INVALID;
-    h->tuning = on && !use_lines(h) ? 1 : 0;   // the column kernels have one shape
+    h->tuning = on ? 1 : 0;   // waits while the column kernels run, which have one shape
     h->tune_i = -1;
     h->tune_tf.clear();
     h->tune_tc.clear();
@@ -3855,7 +3855,7 @@ int dugks_autotune_steps_left(dugks_engine *h, int32_t *steps)
 {
     if (!h || !steps) return DUGKS_ERR_INVALID;
     const int n = std::max((int)h->face_cand.size(), (int)h->cell_cand.size());
-    *steps = h->tuning ? dugks_engine::TUNE_ROUNDS * n - h->tune_i : 0;
+    *steps = h->tuning && !use_lines(h) ? dugks_engine::TUNE_ROUNDS * n - h->tune_i : 0;
     return 0;
 }
 

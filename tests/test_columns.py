@@ -272,3 +272,25 @@ def test_mass_where_one_minus_r_is_small(dt_over_tau):
     print("drift a step", drift, flush=True)
     assert abs(drift) <= 1e-15
     e.close()
+
+
+def test_tuning_waits_for_kernels_that_have_shapes(oracle_lib):
+    """Switched on while the column kernels run, the tuner starts with the first step of other kernels, as
+    dugks_set_face_values(h, 0) brings them."""
+    c = cases.cavity(6, 12)
+    e = Engine(c)
+    e.autotune(True)
+    assert e.autotune_steps_left() == 0
+    e.init_equilibrium()
+    e.step(nsteps=2)
+    e.set_face_values(False)
+    left = e.autotune_steps_left()
+    assert left > 0
+    e.step(nsteps=left)
+    assert e.autotune_steps_left() == 0
+    o = oracle_lib.Oracle(c)
+    o.init_equilibrium()
+    o.step(nsteps=2 + left)
+    assert _off(c, e.macro(), o.macro()) <= 1e-12
+    e.close()
+    o.close()
