@@ -158,3 +158,35 @@ def tetrahedra(n):
             p = [at(b ^ flip) for b in t]
             cells.append([list(f) for f in itertools.combinations(p, 3)])
     return pts, cells
+
+
+def merge(cells, pairs):
+    """Joins cells a, b of each pair over the faces they share."""
+    out = list(cells)
+    for a, b in pairs:
+        fa = {tuple(sorted(f)): f for f in cells[a]}
+        fb = {tuple(sorted(f)): f for f in cells[b]}
+        out[a] = [f for k, f in fa.items() if k not in fb] + [f for k, f in fb.items() if k not in fa]
+        out[b] = None
+    return [c for c in out if c is not None]
+
+
+def pairs(n):
+    """n^3 hexahedra (n even), every other one joined to its neighbour along x: 10 faces."""
+    pts, cells = split_columns(n, n, n, lambda i, j: False)
+    at = lambda i, j, k: (i * n + j) * n + k
+    return pts, merge(cells, [(at(i, j, k), at(i + 1, j, k)) for i in range(0, n, 2) for j in range(n) for k in range(n)
+                              if (i // 2 + j + k) % 2 == 0])
+
+
+def pentagons(n):
+    """The columns of n^3 hexahedra (n even) by twos along x: the first with half of the second, a prism over a
+    pentagon (7 faces), and the other half, a prism over a triangle."""
+    pts, v = grid_points(n, n, n, dz=1.0)
+    cells = []
+    for i, j, k in itertools.product(range(0, n, 2), range(n), range(n)):
+        p, q = (i, j), (i, j + 1)
+        a, b, c, d = (i + 1, j), (i + 2, j), (i + 2, j + 1), (i + 1, j + 1)
+        parts = [[p, a, b, d, q], [b, c, d]] if j % 2 else [[p, a, c, d, q], [a, b, c]]
+        cells += [_prism([v(x, y, k) for x, y in r], [v(x, y, k + 1) for x, y in r]) for r in parts]
+    return pts, cells
