@@ -46,7 +46,6 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <limits>
 #include <mutex>
 #include <new>
 #include <numeric>
@@ -1940,6 +1939,7 @@ struct dugks_engine {
     // velocity columns (lines.h)
     int line_ok = 0;     // the mesh and the velocity set fit the column kernels
     int ntile = 0, line_w = 1;   // tiles; waves per cell
+    void *line_mem = nullptr;   // the device arrays below
     LineRec *rec = nullptr;
     int *titer = nullptr;
     std::vector<int> titer_h;
@@ -2144,6 +2144,27 @@ bool use_lines(const dugks_engine *h) { return h->line_ok && h->face_values && h
 int line_slots(int D, int ns_max)
 {
     return D == 1 ? 2 : (D == 2 ? (ns_max <= 3 ? 3 : 4) : (ns_max <= 4 ? 4 : 6));
+}
+
+// The geometry of every (cell, face) slot of the column kernels, and zeros for the face constants: k_face_fin
+// writes those of the cells' faces, and the loops of k_cell_lines over all slots add nothing in the others.
+__global__ __launch_bounds__(256) void k_line_slots(int D, int ns, size_t n, const int *cs, const Slot *slots, LineGeo *geo,
+                                                    LineFace *face)
+{
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int c = (int)(i / ns), e = cs[c] + (int)(i % ns);
+    const bool has = e < cs[c + 1];
+    const Slot &q = slots[has ? e : cs[c]];
+    const double sgn = q.kind == KIND_NEI ? -1.0 : 1.0;
+    LineGeo g{};
+    g.face = q.face;
+    g.kind = has ? q.kind : KIND_NONE;
+    g.Sl = has ? sgn * q.S[D - 1] : __builtin_nan("");
+    for (int d = 0; d < 3 && has; ++d) g.dC[d] = q.dCs[d];
+    for (int d = 0; d + 1 < D && has; ++d) g.S[d] = sgn * q.S[d];
+    geo[i] = g;
+    face[i] = LineFace{};
 }
 
 // LDS bytes of the column kernels (k_cell_lines: without the new row)
@@ -2974,22 +2995,9 @@ int build(dugks_engine *h, const dugks_case *cs)
     }
     const int lns = line_slots(D, h->ns_max);
     std::vector<int4> fslot(nf, int4{-1, -1, -1, 0});
-    std::vector<LineGeo> lgeo(h->line_ok ? (size_t)nc * lns : 0);
     for (int c = 0; c < nc && h->line_ok; ++c)
-        for (int j = 0; j < lns; ++j) {
-            LineGeo &g = lgeo[(size_t)c * lns + j];
-            std::memset(&g, 0, sizeof g);
-            g.face = sl[cnt[c]].face;
-            g.kind = KIND_NONE;
-            g.Sl = std::numeric_limits<double>::quiet_NaN();
-            if (cnt[c] + j >= cnt[c + 1]) continue;
+        for (int j = 0; j < cnt[c + 1] - cnt[c]; ++j) {
             const Slot &q = sl[cnt[c] + j];
-            const double sgn = q.kind == KIND_NEI ? -1.0 : 1.0;
-            g.face = q.face;
-            g.kind = q.kind;
-            for (int d = 0; d < 3; ++d) g.dC[d] = q.dCs[d];
-            for (int d = 0; d + 1 < D; ++d) g.S[d] = sgn * q.S[d];
-            g.Sl = sgn * q.S[D - 1];
             (q.kind == KIND_NEI ? fslot[q.face].y : fslot[q.face].x) = c * lns + j;
         }
     for (size_t i = 0; i < open_faces.size(); ++i) fslot[open_faces[i]].z = (int)i;
@@ -3110,18 +3118,42 @@ int build(dugks_engine *h, const dugks_case *cs)
         (r = upload(h, h->fx, fxs.data(), nf)) || (r = upload(h, h->cst, cst.data(), nc)) ||
         (r = upload(h, h->corder, corder.data(), nc)) || (r = upload(h, h->forder, forder.data(), nf)) || (r = upload(h, h->wfslot, wfslot.data(), nw)))
         return r;
-    if (h->line_ok &&
-        ((r = dalloc(h, &h->img_slot, img_slot.size())) || (r = upload(h, h->img_slot, img_slot.data(), img_slot.size())) ||
-         (r = dalloc(h, &h->rec, recs.size())) || (r = upload(h, h->rec, recs.data(), recs.size())) ||
-         (r = dalloc(h, &h->titer, h->titer_h.size())) || (r = upload(h, h->titer, h->titer_h.data(), h->titer_h.size())) ||
-         (r = dalloc(h, &h->lgeo, lgeo.size())) || (r = upload(h, h->lgeo, lgeo.data(), lgeo.size())) ||
-         (r = dalloc(h, &h->spart, (size_t)nc * lns * NMom<3>::v)) ||
-         (r = dalloc(h, &h->opart, open_faces.size() * NMom<3>::v)) || (r = dalloc(h, &h->lface, (size_t)nc * lns)) || (r = dalloc(h, &h->lcell, (size_t)nc)) ||
-         (r = dalloc(h, &h->fslot, nf)) || (r = upload(h, h->fslot, fslot.data(), nf))))
-        return r;
-    // k_face_fin writes the slots of the cells' faces; the others stay 0, so that the loops of
-    // k_cell_lines over all slots add nothing there
-    if (h->line_ok) HIPCHK(h, hipMemsetAsync(h->lface, 0, sizeof(LineFace) * (size_t)nc * lns, h->stream));
+    if (h->line_ok) {
+        // the arrays of the column kernels in one allocation, those made here first
+        const size_t slots = (size_t)nc * lns;
+        size_t bytes = 0;
+        auto place = [&](size_t n) {
+            const size_t at = bytes;
+            bytes += (n + 255) / 256 * 256;
+            return at;
+        };
+        const size_t n_img = sizeof(int) * img_slot.size(), n_rec = sizeof(LineRec) * recs.size(),
+                     n_it = sizeof(int) * h->titer_h.size(), n_fs = sizeof(int4) * nf;
+        const size_t img = place(n_img), rec = place(n_rec), it = place(n_it), fs = place(n_fs), made = bytes;
+        const size_t geo = place(sizeof(LineGeo) * slots), face = place(sizeof(LineFace) * slots),
+                     cell = place(sizeof(LineCell) * nc), sp = place(sizeof(double) * NMom<3>::v * slots),
+                     op = place(sizeof(double) * NMom<3>::v * open_faces.size());
+        if ((r = dallocb(h, &h->line_mem, bytes))) return r;
+        std::vector<char> host(made, 0);
+        std::memcpy(&host[img], img_slot.data(), n_img);
+        std::memcpy(&host[rec], recs.data(), n_rec);
+        std::memcpy(&host[it], h->titer_h.data(), n_it);
+        std::memcpy(&host[fs], fslot.data(), n_fs);
+        char *m = (char *)h->line_mem;
+        HIPCHK(h, hipMemcpy(m, host.data(), made, hipMemcpyHostToDevice));
+        h->img_slot = (int *)(m + img);
+        h->rec = (LineRec *)(m + rec);
+        h->titer = (int *)(m + it);
+        h->fslot = (int4 *)(m + fs);
+        h->lgeo = (LineGeo *)(m + geo);
+        h->lface = (LineFace *)(m + face);
+        h->lcell = (LineCell *)(m + cell);
+        h->spart = (double *)(m + sp);
+        h->opart = (double *)(m + op);
+        hipLaunchKernelGGL(k_line_slots, dim3((slots + 255) / 256), dim3(256), 0, h->stream, D, lns, slots, h->cs, h->slots,
+                           h->lgeo, h->lface);
+        HIPCHK(h, hipGetLastError());
+    }
     if (nw && (r = upload(h, h->wall, wc.data(), nw))) return r;
     if (nw && ((r = dalloc(h, &h->bpress, nw)) || (r = upload(h, h->bpress, wpress.data(), nw)))) return r;
     h->nopen = (int)open_faces.size();
@@ -3174,7 +3206,7 @@ void release(dugks_engine *h)
     dfree(h->ctau); dfree(h->frho); dfree(h->fU); dfree(h->fT); dfree(h->fq); dfree(h->feq);
     dfree(h->wall); dfree(h->wexp); dfree(h->qwall); dfree(h->swall); dfree(h->fx); dfree(h->cst);
     dfree(h->corder); dfree(h->forder); dfree(h->fpart); dfree(h->cpart); dfree(h->mxf); dfree(h->wallf);
-    dfree(h->rec); dfree(h->titer); dfree(h->img_slot); dfree(h->lgeo); dfree(h->spart); dfree(h->opart); dfree(h->lface); dfree(h->lcell); dfree(h->fslot);
+    dfree(h->line_mem);
     for (int i = 0; i < 2; ++i) {
         dfree(h->gb[i]); dfree(h->hb[i]);
         h->gB[i] = h->hB[i] = nullptr;
