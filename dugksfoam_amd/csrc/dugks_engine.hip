@@ -1943,7 +1943,11 @@ struct dugks_engine {
     LineRec *rec = nullptr;
     int *titer = nullptr;
     std::vector<int> titer_h;
-    int nvp_img = 0;     // padded velocity count of a state image's rows
+    // row orders (reference velocity of every slot, -1 padding): sign-sorted, also that of a state image's rows,
+    // and the columns; the rows are in the second while the column kernels run
+    std::vector<int> order_img, order_col;
+    int columns = 0;     // 1: rows in column order
+    int nvp_img = 0;     // slots of a sign-sorted row
     int *img_slot = nullptr;
     LineGeo *lgeo = nullptr;
     double *spart = nullptr, *opart = nullptr;
@@ -2465,6 +2469,15 @@ void shape_candidates(dugks_engine *h)
     h->nbc_cap = h->nb_cap = std::max(h->nb_cap, h->nbc_cap);
 }
 
+// Shapes for rows of n slots and their padding
+void row_shapes(dugks_engine *h, int n)
+{
+    choose_blocks(n, h->nt, h->nib, h->nvb, h->nvp);
+    h->vb = h->nt * h->nib;
+    h->niter = h->nvb * h->nib;
+    shape_candidates(h);
+}
+
 // Velocity columns of the tensor set (lines.h): the lanes of every tile, the iterations before each
 // tile, and the velocity (reference index, -1 padding) of every slot of a row.  A column has fixed
 // (x, y) (3-D) or x (2-D) and runs over every m-th velocity of the last axis.  Columns are ordered by
@@ -2641,6 +2654,31 @@ int kind_of(int patch_type)
     case DUGKS_PATCH_ZEROGRADIENT: return KIND_ZG;
     default: return KIND_FAR;   // far field, fixed, pressure inlet / outlet
     }
+}
+
+// The device's tables of a row order: packed axis indices, and the mirrored velocities (symmXtgID /
+// symmYtgID / symmZtgID, fvDVM.C:152-166, 183-195).
+int upload_rows(dugks_engine *h, const std::vector<int> &order)
+{
+    const int D = h->D, nxi = h->nxi, nvp = h->nvp, ny = D >= 2 ? nxi : 1, nz = D == 3 ? nxi : 1;
+    std::vector<uint32_t> vidx(nvp, VPAD), mir(3 * (size_t)nvp);
+    std::vector<int> inv(h->nv);
+    for (int k = 0; k < nvp; ++k) {
+        for (int a = 0; a < 3; ++a) mir[(size_t)a * nvp + k] = (uint32_t)k;
+        if (order[k] >= 0) inv[order[k]] = k;
+    }
+    for (int k = 0; k < nvp; ++k) {
+        const int r = order[k];
+        if (r < 0) continue;
+        const int ix = r % nxi, iy = D >= 2 ? (r / nxi) % nxi : 0, iz = D == 3 ? r / (nxi * nxi) : 0;
+        vidx[k] = (uint32_t)(ix | (iy << 8) | (iz << 16));
+        mir[k] = (uint32_t)inv[(iz * ny + iy) * nxi + (nxi - 1 - ix)];
+        mir[(size_t)nvp + k] = (uint32_t)inv[(iz * ny + (ny - 1 - iy)) * nxi + ix];
+        mir[2 * (size_t)nvp + k] = (uint32_t)inv[((nz - 1 - iz) * ny + iy) * nxi + ix];
+    }
+    h->perm = order;
+    if (int r = upload(h, h->vidx, vidx.data(), nvp)) return r;
+    return upload(h, h->mir, mir.data(), 3 * (size_t)nvp);
 }
 
 int build(dugks_engine *h, const dugks_case *cs)
@@ -2875,7 +2913,6 @@ int build(dugks_engine *h, const dugks_case *cs)
     if (h->nax > NAXMAX) return fail(h, DUGKS_ERR_UNSUPPORTED, "velocity table too large");
     const int nv = h->nv;
     std::vector<double> rx(nv), ry(nv), rz(nv);
-    std::vector<int> rid(nv);
     {
         int i = 0;
         const double *X = cs->xi;
@@ -2884,20 +2921,17 @@ int build(dugks_engine *h, const dugks_case *cs)
                 for (int iy = 0; iy < nxi; ++iy)
                     for (int ix = 0; ix < nxi; ++ix) {
                         rx[i] = X[ix]; ry[i] = X[iy]; rz[i] = X[iz];
-                        rid[i] = ix | (iy << 8) | (iz << 16);
                         ++i;
                     }
         } else if (D == 2) {
             for (int iy = 0; iy < nxi; ++iy)
                 for (int ix = 0; ix < nxi; ++ix) {
                     rx[i] = X[ix]; ry[i] = X[iy]; rz[i] = 0.0;
-                    rid[i] = ix | (iy << 8);
                     ++i;
                 }
         } else {
             for (int ix = 0; ix < nxi; ++ix) {
                 rx[i] = X[ix]; ry[i] = 0.0; rz[i] = 0.0;
-                rid[i] = ix;
                 ++i;
             }
         }
@@ -2913,12 +2947,13 @@ int build(dugks_engine *h, const dugks_case *cs)
     // ---- row layout ----
     // Sign-sorted velocities, or (meshes and options of the column kernels) the slots of their tiles,
     // where the face values fit as they have to for face-value mode to be the default.
-    choose_blocks(nv, h->nt, h->nib, h->nvb, h->nvp);
+    row_shapes(h, nv);
     h->nvp_img = h->nvp;
+    h->order_img = order;
+    h->order_img.resize(h->nvp, -1);
     h->ns_max = 0;
     for (int c = 0; c < nc; ++c) h->ns_max = std::max(h->ns_max, cnt[c + 1] - cnt[c]);
     std::vector<LineRec> recs;
-    std::vector<int> slot_ref(order);
     h->titer_h.assign(1, 0);
     {
         const char *fm = std::getenv("DUGKS_FACE_MFMA"), *fl = std::getenv("DUGKS_FACE_PASS_LEGACY"),
@@ -2935,15 +2970,15 @@ int build(dugks_engine *h, const dugks_case *cs)
             h->line_ok = es * nf <= 0.5 * ((double)fr - 2.0 * es * ((double)nc + h->nw) - 2048.0 * ((double)nc + nf));
         }
         if (h->line_ok) {
+            const int cap = h->nb_cap;
             h->ntile = (int)h->titer_h.size() - 1;
-            slot_ref = refs;
-            choose_blocks((int)refs.size(), h->nt, h->nib, h->nvb, h->nvp);
+            h->columns = 1;
+            row_shapes(h, (int)refs.size());
+            h->order_col = refs;
+            h->order_col.resize(h->nvp, -1);
+            h->nbc_cap = h->nb_cap = std::max(h->nb_cap, cap);   // for the kernels of either order
         }
     }
-    slot_ref.resize(h->nvp, -1);
-    h->vb = h->nt * h->nib;
-    h->niter = h->nvb * h->nib;
-    shape_candidates(h);
     if (h->nt <= 0 || h->nt > MAXNT || h->nvp < nv)
         return fail(h, DUGKS_ERR_UNSUPPORTED, "velocity blocking failed");
     // one dispatch holds at most 2^32 - 1 work-items per grid dimension
@@ -2981,16 +3016,11 @@ int build(dugks_engine *h, const dugks_case *cs)
         cst[c] = t;
     }
     const int nvp = h->nvp;
-    std::vector<uint32_t> vidx(nvp, VPAD);
-    h->perm = slot_ref;
-    std::vector<int> img_slot(h->nvp_img, -1);   // state image: sign-sorted velocity -> slot
-    {
+    std::vector<int> img_slot(h->nvp_img, -1);   // sign-sorted slot -> column slot
+    if (h->line_ok) {
         std::vector<int> slot(nv);
         for (int k = 0; k < nvp; ++k)
-            if (slot_ref[k] >= 0) {
-                vidx[k] = (uint32_t)rid[slot_ref[k]];
-                slot[slot_ref[k]] = k;
-            }
+            if (h->order_col[k] >= 0) slot[h->order_col[k]] = k;
         for (int k = 0; k < nv; ++k) img_slot[k] = slot[order[k]];
     }
     const int lns = line_slots(D, h->ns_max);
@@ -3001,24 +3031,6 @@ int build(dugks_engine *h, const dugks_case *cs)
             (q.kind == KIND_NEI ? fslot[q.face].y : fslot[q.face].x) = c * lns + j;
         }
     for (size_t i = 0; i < open_faces.size(); ++i) fslot[open_faces[i]].z = (int)i;
-    // mirrored velocities (symmXtgID / symmYtgID / symmZtgID, fvDVM.C:152-166, 183-195) in device order
-    std::vector<uint32_t> mir(3 * (size_t)nvp);
-    {
-        std::vector<int> inv(nv);
-        for (int k = 0; k < nvp; ++k)
-            if (h->perm[k] >= 0) inv[h->perm[k]] = k;
-        for (int k = 0; k < nvp; ++k)
-            for (int a = 0; a < 3; ++a) mir[(size_t)a * nvp + k] = (uint32_t)k;
-        for (int k = 0; k < nvp; ++k) {
-            const int r = h->perm[k];
-            if (r < 0) continue;
-            const int ix = r % nxi, iy = D >= 2 ? (r / nxi) % nxi : 0, iz = D == 3 ? r / (nxi * nxi) : 0;
-            const int ny = D >= 2 ? nxi : 1, nz = D == 3 ? nxi : 1;
-            mir[k] = (uint32_t)inv[(iz * ny + iy) * nxi + (nxi - 1 - ix)];
-            mir[(size_t)nvp + k] = (uint32_t)inv[(iz * ny + (ny - 1 - iy)) * nxi + ix];
-            mir[2 * (size_t)nvp + k] = (uint32_t)inv[((nz - 1 - iz) * ny + iy) * nxi + ix];
-        }
-    }
     std::vector<double> axis(h->nax), axw(h->nax);
     for (int a = 0; a < D; ++a)
         for (int i = 0; i < nxi; ++i) {
@@ -3111,7 +3123,7 @@ int build(dugks_engine *h, const dugks_case *cs)
             h->hB[i] = (char *)h->hb[i] + row;
         }
     }
-    if ((r = upload(h, h->vidx, vidx.data(), nvp)) || (r = upload(h, h->mir, mir.data(), 3 * (size_t)nvp)) || (r = upload(h, h->axw, axw.data(), h->nax)) ||
+    if ((r = upload_rows(h, h->columns ? h->order_col : h->order_img)) || (r = upload(h, h->axw, axw.data(), h->nax)) ||
         (r = upload(h, h->axis, axis.data(), h->nax)) || (r = upload(h, h->cs, cnt.data(), nc + 1)) ||
         (r = upload(h, h->slots, sl.data(), nslot)) || (r = upload(h, h->cV, cs->V, nc)) ||
         (r = upload(h, h->ccase, ccase.data(), nc)) || (r = upload(h, h->muc, muc.data(), h->n_cases)) ||
@@ -3385,8 +3397,8 @@ int step_impl(dugks_engine *h, const double *dtc, int nsteps)
     return r;
 }
 
-// Rows of the current state <-> rows of a state image (sign-sorted velocities, nvp_img a row), for the
-// column layout.  The other ping-pong side, which holds nothing between steps, stages them.
+// Rows in column order <-> sign-sorted rows (nvp_img slots, those of a state image), from one ping-pong side to
+// the other, which holds nothing between steps.
 template <typename TS>
 __global__ __launch_bounds__(256) void k_image(TS *img, TS *rows, const int *slot, int nimg, int nvp, int save)
 {
@@ -3400,22 +3412,66 @@ __global__ __launch_bounds__(256) void k_image(TS *img, TS *rows, const int *slo
 
 void image_rows(dugks_engine *h, void *img, void *rows, int save)
 {
-    const int n = h->nc + (h->nw ? h->nw : 1);
+    const int n = h->nc + (h->nw ? h->nw : 1), nvp = (int)h->order_col.size();
     if (h->storage == DUGKS_STORAGE_FP32)
-        hipLaunchKernelGGL((k_image<float>), dim3(n), dim3(256), 0, h->stream, (float *)img, (float *)rows, h->img_slot, h->nvp_img, h->nvp, save);
+        hipLaunchKernelGGL((k_image<float>), dim3(n), dim3(256), 0, h->stream, (float *)img, (float *)rows, h->img_slot, h->nvp_img, nvp, save);
     else
-        hipLaunchKernelGGL((k_image<double>), dim3(n), dim3(256), 0, h->stream, (double *)img, (double *)rows, h->img_slot, h->nvp_img, h->nvp, save);
+        hipLaunchKernelGGL((k_image<double>), dim3(n), dim3(256), 0, h->stream, (double *)img, (double *)rows, h->img_slot, h->nvp_img, nvp, save);
 }
 
-// Zeros a ping-pong side that staged an image.  The column kernels write the nv velocities of a row only; what
-// reads the padding gives it weight 0, so it has to be finite (dugks_init_equilibrium and the conversion
-// that follows write all of a row).
+// Zeros a ping-pong side.  The column kernels write the nv velocities of a row only; what reads the padding
+// gives it weight 0, so it has to be finite: after a side held sign-sorted rows it is cleared
+// (dugks_init_equilibrium and the conversion that follows write all of a row).
 int clear_side(dugks_engine *h, int side)
 {
-    const size_t bytes = ((size_t)h->nc + (h->nw ? h->nw : 1)) * h->nvp * ts_size(h);
+    const size_t bytes = ((size_t)h->nc + (h->nw ? h->nw : 1)) * h->order_col.size() * ts_size(h);
     HIPCHK(h, hipMemsetAsync(h->gb[side], 0, bytes, h->stream));
     if (h->has_h) HIPCHK(h, hipMemsetAsync(h->hb[side], 0, bytes, h->stream));
     return 0;
+}
+
+__global__ __launch_bounds__(256) void k_row_stride(CellSt *st, int n, int from, int to)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n * MAXS) {
+        int64_t &o = st[i / MAXS].off[i % MAXS];
+        o = o / from * to;
+    }
+}
+
+// Brings the rows into the order of the kernels that run: column order for the column kernels, sign-sorted for
+// the others, where a wave's velocities lie on one side of an axis-aligned face (rebuilding kernels, 60^2
+// cells of 41^2 velocities: 338 us a step, 431 over column rows; 24^3 of 24^3: 9.5 and 10.1 ms).
+int set_rows(dugks_engine *h, int columns)
+{
+    if (!h->line_ok || columns == h->columns) return 0;
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    const int cur = h->cur, side = 1 - cur;
+    if (columns)
+        if (int r = clear_side(h, side)) return r;
+    for (int i = 0; i < (h->has_h ? 2 : 1); ++i) {
+        void **b = i ? h->hb : h->gb;
+        image_rows(h, b[columns ? cur : side], b[columns ? side : cur], !columns);
+    }
+    HIPCHK(h, hipGetLastError());
+    if (columns)
+        if (int r = clear_side(h, cur)) return r;
+    const int from = h->nvp, cap = h->nb_cap;
+    row_shapes(h, columns ? (int)h->order_col.size() : h->nv);
+    h->nbc_cap = h->nb_cap = cap;
+    hipLaunchKernelGGL(k_row_stride, dim3(((size_t)h->nc * MAXS + 255) / 256), dim3(256), 0, h->stream, h->cst, h->nc, from, h->nvp);
+    HIPCHK(h, hipGetLastError());
+    for (int i = 0; i < 2; ++i) {
+        h->gB[i] = (char *)h->gb[i] + (size_t)h->nc * h->nvp * ts_size(h);
+        if (h->has_h) h->hB[i] = (char *)h->hb[i] + (size_t)h->nc * h->nvp * ts_size(h);
+    }
+    h->cur = side;
+    h->columns = columns;
+    h->tune_i = -1;
+    h->tune_tf.clear();
+    h->tune_tc.clear();
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    return upload_rows(h, columns ? h->order_col : h->order_img);
 }
 
 const int64_t STATE_MAGIC = 0x44554b5331LL;  // "DUKS1"
@@ -3490,6 +3546,7 @@ int dugks_create(const dugks_case *cs, dugks_engine **out)
         // DUGKS_FUSE_S1=0 keeps k_cell_fin and k_cell_s1 as kernels of their own
         const char *f1 = std::getenv("DUGKS_FUSE_S1");
         h->fuse_s1 = f1 && !std::atoi(f1) ? 0 : 1;
+        if (!r) r = set_rows(h, use_lines(h));
     }
     if (!r) {
         // this device's copy of the dugks_get_df_noalloc scratch; a failure is reported by that
@@ -3783,8 +3840,8 @@ int dugks_save_state(dugks_engine *h, void *buf, int64_t bytes)
     p += sizeof hdr;
     const size_t es = ts_size(h);
     const size_t row = (size_t)h->nc * h->nvp_img * es, brow = (size_t)(h->nw ? h->nw : 1) * h->nvp_img * es;
-    const int side = h->line_ok ? 1 - h->cur : h->cur;
-    if (h->line_ok) {
+    const int side = h->columns ? 1 - h->cur : h->cur;
+    if (h->columns) {
         image_rows(h, h->gb[side], h->gb[h->cur], 1);
         if (h->has_h) image_rows(h, h->hb[side], h->hb[h->cur], 1);
         HIPCHK(h, hipGetLastError());
@@ -3795,7 +3852,7 @@ int dugks_save_state(dugks_engine *h, void *buf, int64_t bytes)
     if (h->has_h) { HIPCHK(h, hipMemcpy(p, hr, row, hipMemcpyDeviceToHost)); p += row; }
     HIPCHK(h, hipMemcpy(p, gr + row, brow, hipMemcpyDeviceToHost)); p += brow;
     if (h->has_h) { HIPCHK(h, hipMemcpy(p, hr + row, brow, hipMemcpyDeviceToHost)); p += brow; }
-    if (h->line_ok)
+    if (h->columns)
         if (int rr = clear_side(h, side)) return rr;
     const size_t nc = h->nc;
     HIPCHK(h, hipMemcpy(p, h->crho, 8 * nc, hipMemcpyDeviceToHost)); p += 8 * nc;
@@ -3828,13 +3885,13 @@ int dugks_load_state(dugks_engine *h, const void *buf, int64_t bytes)
     HIPCHK(h, hipStreamSynchronize(h->stream));
     const size_t es = ts_size(h);
     const size_t row = (size_t)h->nc * h->nvp_img * es, brow = (size_t)(h->nw ? h->nw : 1) * h->nvp_img * es;
-    const int side = h->line_ok ? 1 - h->cur : h->cur;
+    const int side = h->columns ? 1 - h->cur : h->cur;
     char *gr = (char *)h->gb[side], *hr = (char *)h->hb[side];
     HIPCHK(h, hipMemcpy(gr, p, row, hipMemcpyHostToDevice)); p += row;
     if (h->has_h) { HIPCHK(h, hipMemcpy(hr, p, row, hipMemcpyHostToDevice)); p += row; }
     HIPCHK(h, hipMemcpy(gr + row, p, brow, hipMemcpyHostToDevice)); p += brow;
     if (h->has_h) { HIPCHK(h, hipMemcpy(hr + row, p, brow, hipMemcpyHostToDevice)); p += brow; }
-    if (h->line_ok) {
+    if (h->columns) {
         image_rows(h, gr, h->gb[h->cur], 0);
         if (h->has_h) image_rows(h, hr, h->hb[h->cur], 0);
         HIPCHK(h, hipGetLastError());
@@ -3917,7 +3974,7 @@ int dugks_set_face_values(dugks_engine *h, int32_t on)
     HIPCHK(h, hipSetDevice(h->device));
     HIPCHK(h, hipStreamSynchronize(h->stream));
     if (on && !h->fvg) {
-        const size_t bytes = (size_t)h->nf * h->nvp * ts_size(h);
+        const size_t bytes = (size_t)h->nf * (h->line_ok ? h->order_col.size() : (size_t)h->nvp) * ts_size(h);
         int r;
         if ((r = dallocb(h, &h->fvg, bytes))) return r;
         if (h->has_h && (r = dallocb(h, &h->fvh, bytes))) {
@@ -3929,9 +3986,10 @@ int dugks_set_face_values(dugks_engine *h, int32_t on)
         dfree(h->fvh);
     }
     h->face_values = on ? 1 : 0;
-    default_cell_shape(h);
     drop_graphs(h);
-    return 0;
+    const int r = set_rows(h, use_lines(h));
+    default_cell_shape(h);
+    return r;
 }
 
 int dugks_get_launch(dugks_engine *h, int32_t *nt, int32_t *nib, int32_t *n_blocks, int32_t *nv_padded)

@@ -294,3 +294,52 @@ def test_tuning_waits_for_kernels_that_have_shapes(oracle_lib):
     assert _off(c, e.macro(), o.macro()) <= 1e-12
     e.close()
     o.close()
+
+
+@pytest.mark.parametrize("which,storage", [("2d", "fp64"), ("2d", "fp32"), ("cyclic_K2", "fp64"), ("1d", "fp64"),
+                                           ("3d_K2", "fp32"), ("prisms", "fp64")])
+def test_rows_follow_the_kernels(which, storage, oracle_lib, monkeypatch):
+    """Without face values the engine is the one that never had columns: the same shapes and bits.  Switched to
+    and fro between steps it keeps its state: as far from the oracle as without (3 + 2 + 2 steps)."""
+    c = {"2d": lambda: cases.cavity(5, 41), "cyclic_K2": lambda: cases.channel(8, 4, 2.0, 1.0, nv=11, K=2),
+         "1d": lambda: cases.fourier_flow(9, nv=63), "3d_K2": lambda: cases.cavity(3, 9, dim=3, K=2),
+         "prisms": lambda: _box(3, _strip(3), "prisms", 7)}[which]()
+    tol = 1e-12 if storage == "fp64" else 1e-6
+    e = Engine(c, storage=storage)
+    columns = e.blocks()
+    e.set_face_values(False)
+    monkeypatch.setenv("DUGKS_FACE_MFMA", "0")
+    r = Engine(c, storage=storage)
+    monkeypatch.delenv("DUGKS_FACE_MFMA")
+    r.set_face_values(False)
+    assert e.blocks() == r.blocks() and e.cell_blocks() == r.cell_blocks()
+    for x in (e, r):
+        x.init_equilibrium()
+        x.step(nsteps=3)
+    cells = np.arange(c.n_cells, dtype=np.int32)
+    for a, b in ((e.macro(), r.macro()), (e.face_macro(), r.face_macro())):
+        assert all(np.array_equal(a[k], b[k]) for k in a)
+    assert all(np.array_equal(a, b) for a, b in zip(e.df(cells), r.df(cells)))
+    e.set_face_values(True)
+    assert _on_columns(e) and e.blocks() == columns
+    assert all(np.array_equal(a, b) for a, b in zip(e.df(cells), r.df(cells)))
+    img = r.save_state()
+    e.load_state(img)
+    assert all(np.array_equal(a, b) for a, b in zip(e.df(cells), r.df(cells)))
+    e.step(nsteps=2)
+    e.set_face_values(False)
+    e.step(nsteps=2)
+    o = oracle_lib.Oracle(c)
+    o.init_equilibrium()
+    o.step(nsteps=7)
+    assert _off(c, e.macro(), o.macro()) <= tol
+    assert _off(c, e.face_macro(), o.face_macro()) <= tol
+    e.load_state(img)
+    assert all(np.array_equal(a, b) for a, b in zip(e.df(cells), r.df(cells)))
+    for x in (e, r):
+        x.step(nsteps=2)
+    a, b = e.macro(), r.macro()
+    assert all(np.array_equal(a[k], b[k]) for k in a)
+    for x in (e, r):
+        x.close()
+    o.close()
