@@ -2493,9 +2493,11 @@ void row_shapes(dugks_engine *h, int n)
 //     past 13 (16^3 velocities, 30^3 cells: 2.97 ms with 1 wave of 64 iterations, 2.74 with 2; 24^3, 24^3:
 //     5.30 with 1 wave of 216, 4.44 with 3), a third where all waves run at once, each phase
 //     together (60^2 cells of 41^2: 304 us with 1, 247 with 2);
-//   - all cells cost that times the rounds of waves the device needs (48^2 cells of 35^2 velocities: 150,
-//     160 and 140 us with 1, 2 and 3 waves a cell, 1, 2 and 2 rounds); past a few rounds the last one's
-//     idle half is what counts.
+//   - all cells cost that times the rounds of waves the device needs, of which the last, filled to a fraction
+//     f, takes (1 + f) / 2: few waves on a CU run faster than many (48^2 cells of 35^2 velocities: 150, 160 and
+//     140 us with 1, 2 and 3 waves a cell, 0.56, 1.1 and 1.7 rounds; 4624 cells of 24^2 FP32: 128 us with 1 wave,
+//     142 with 3 of a third the length, 1.1 and 3.4 rounds).  Over 220 sizes and every m and w the choice is 1.0 %
+//     slower than the best one on average, with whole rounds 2.2 %.
 // At most 4 waves a cell: 48^3 cells of 24^3 velocities take 34.4 ms with 3, 49.7 with 5.
 constexpr double TILE_COST = 0.8, MIX_COST = 0.1, WAVE_COST = 2.0;
 // The columns are built once, for the m chosen; the search goes over runs of columns of one length and class.
@@ -2604,7 +2606,8 @@ void velocity_columns(int D, int nxi, const double *xi, int nc, int slots, int l
             double busy[4] = {WAVE_COST, WAVE_COST, WAVE_COST, WAVE_COST};
             for (size_t t = 0; t < tile.size(); ++t) busy[t % w] += tile[t];
             const double b = *std::max_element(busy, busy + w);
-            const double x = (double)nc * w / slots, rounds = x < 3 ? std::ceil(x) : x + 0.5;
+            const double x = (double)nc * w / slots, full = std::floor(x);
+            const double rounds = full + (x > full ? 0.5 + 0.5 * (x - full) : 0.0);
             const double lone = 0.35 * std::min(1.0, std::max(0.0, (b - 20) / 13)), tail = 0.1 * std::max(0.0, std::log2(b / 13));
             const double cost = rounds * b * (1 + (x <= 1 ? lone : tail));
             if (best_cost < 0 || cost < best_cost) {
