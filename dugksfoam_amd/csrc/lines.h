@@ -216,7 +216,7 @@ DEVI Column<D> column_at(const P<TS> &p, const LineRec &r, const double *vt)
 
 // The loop-axis table in LDS: LT doubles per axis position.
 //   [0] coordinate, [1..4] w (z - Ur)^m, m = 0..3, [5] FP32 row-offset factor, [6] cell equilibrium's
-//   exp factor, [8 + j] face j's exp factor
+//   exp factor, [7] index in the per-axis tables, [8 + j] face j's exp factor
 // One address and immediate offsets serve every entry of an iteration.
 template <int NS>
 constexpr int line_lt()
@@ -656,7 +656,8 @@ DEVI void line_geq(double z, double invRT, double B, double qz, double RT, doubl
     heq = H ? fma(pc, fma(Pv, kc, kc2K), kc) * (gB * RT) : 0.0;   // kc2K = 2 kc - 2 K
 }
 
-// Cell equilibrium's exp factors: fixed axes in tabC, the loop axis in entry 6 of the axis table.
+// Cell equilibrium's exp factors: fixed axes in tabC, the loop axis in entry 6 of the axis table, and its index
+// in entry 7.
 template <int LT, typename TS>
 DEVI void stage_cell_exp(const P<TS> &p, int la0, const double *U, double invRT, double *tabC, double *tab)
 {
@@ -664,8 +665,12 @@ DEVI void stage_cell_exp(const P<TS> &p, int la0, const double *U, double invRT,
         const int ax = t / p.nxi;
         const double u = U[ax] - p.axis[t - ax * p.nxi];
         const double e = exp(-(u * u) * (0.5 * invRT));
-        if (t >= la0) tab[(t - la0) * LT + 6] = e;
-        else tabC[t] = e;
+        if (t >= la0) {
+            tab[(t - la0) * LT + 6] = e;
+            tab[(t - la0) * LT + 7] = t;
+        } else {
+            tabC[t] = e;
+        }
     }
 }
 
@@ -908,8 +913,7 @@ __global__ __launch_bounds__(LINE_MAXNT) __attribute__((amdgpu_waves_per_eu(D ==
                     // field operation, 880-881), the outgoing ones once more (905-920)
                     const bool all = kind == KIND_OWN || kind == KIND_NEI || kind == KIND_CYC || kind == KIND_SPL;
                     if (kind == KIND_WALL && !(so > 0)) {
-                        const int l = (int)((LDS_AS const double *)e - (LDS_AS const double *)tab) / LT;
-                        g = tabW[(la0 + l) * NS + j];
+                        g = tabW[(int)e[7] * NS + j];
                         if (D >= 2) g *= tabW[col.ix * NS + j];
                         if (D == 3) g *= tabW[(nxi + col.iy) * NS + j];
                         if (H) h = g * (p.R * cptr(p.feq)[S.face].pad[0]) * p.kc;
