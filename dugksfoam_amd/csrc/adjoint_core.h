@@ -92,8 +92,8 @@ struct CP {
 
 // Rows of a point's velocities on chip (the phases that pass over them again would read them back through
 // the L2, and a forward step whose reverse does not follow need not write its face values at all; 16000
-// faces of 32^2 velocities: k_face 467 -> 306 us with the scalar loads of CP and one upwind row, k_face_adj
-// 374 -> 294): an executor with local_rows keeps row i (nv values, each
+// faces of 32^2 velocities: k_face 463 -> 316 us with the scalar loads of CP and one upwind row, k_face_adj
+// 371 -> 296): an executor with local_rows keeps row i (nv values, each
 // written and read by the worker that owns its velocity) there, others in the given work array.
 template <class X, class = void>
 struct has_rows : std::false_type {};
@@ -674,7 +674,7 @@ ADJ_HD void face_fwd(X &x, const AP &p, int f, const double *mac, const double *
 
 // S8 (discreteVelocity.C:934-978) and S9 (fvDVM.C:597-728) of one cell into state nx; with s1 also S1
 // of the next step, over this step's gbar+ of the cell, from the row that is at hand (8000 cells of 32^2
-// velocities: 201 + 55 us as two kernels, 224 as one; memory bound).
+// velocities: 202 + 55 us as two kernels, 229 as one; memory bound).
 template <class X>
 ADJ_HD void cell_fwd(X &x, const AP &p, St s, int c, double *gp, double *hp, const double *gr, const double *hr,
                      St nx, bool s1)
@@ -993,7 +993,7 @@ ADJ_HD void recon_adj(X &x, const AP &p, int c, const double *abf, const double 
 // Reverse of the least-squares gradient gathered at one cell (adds to the adjoint of gbar+, writes the
 // adjoint of the lagged rows G^n of its wall faces), of S1, then the adjoint of the state's macros (S9 of
 // the previous step) folded into the distributions: writes the adjoint of g~^n, h~^n.  One kernel: the
-// adjoint of gbar+ stays on chip between its parts (8000 cells of 32^2 velocities: 231 + 186 -> 292 us, bound
+// adjoint of gbar+ stays on chip between its parts (8000 cells of 32^2 velocities: 227 + 185 -> 294 us, bound
 // by the latency that 3 waves a SIMD leave; held to fewer registers the sums spill, 397 us).
 template <class X>
 ADJ_HD void grad_s1_adj(X &x, const AP &p, St s, int c, const double *ag1, const double *ah1, const double *agg,

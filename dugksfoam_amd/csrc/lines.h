@@ -9,7 +9,7 @@
 // A lane that takes any velocity and rebuilds all of it is bound by its vector instructions, about
 // three times as many; and the face moments ride along in the pass that forms the face values instead
 // of reading them back from HBM.  A step before (k_face_values, k_face_moments, k_cell) and now, ms:
-//   48^3 cells, 24^3 velocities, FP64    46.9  35.8      20000 triangles, 64^2, FP64    5.77  4.48
+//   48^3 cells, 24^3 velocities, FP64    46.9  35.9      20000 triangles, 64^2, FP64    5.77  4.48
 //   48^3 cells, 24^3 velocities, FP32    36.6  28.2      64 cavities, 28^2, FP64        6.19  5.16
 //   21^3 cells, 13^3, g and h, FP64      1.77  1.11      60^2 cells, 41^2, FP64        0.310 0.266
 //
@@ -285,7 +285,7 @@ DEVI double col_off(double mo, const double *e, double pre)
 // k_face_moments_mx and k_face_moments).  Every face value is written by its upwind cell, with the
 // selection of k_face_values; the cell's share of each face's moments (the values it wrote) is
 // summed about the cell's previous velocity and left in spart[cell NS + face], one record each.
-// Bound by memory at 3-D sizes (48^3 x 24^3 FP64: 16.1 ms against 15.1 + 6.9 of the two passes), by
+// Bound by memory at 3-D sizes (48^3 x 24^3 FP64: 16.3 ms, 5.3 TB/s, against 15.1 + 6.9 of the two passes), by
 // latency and vector issue at a few thousand cells.  The open faces ride in the first workgroups: alone
 // they are one short kernel of few waves (75 x 25 cells: 13 us of a 110 us step).
 // ---------------------------------------------------------------------------------------------
@@ -730,8 +730,8 @@ DEVI void line_s1(const P<TS> &p, int c, const CellEq &e, const double *tabC, co
 
 // ---------------------------------------------------------------------------------------------
 // k_cell_lines: S7 face relaxation, S8 update and S9 cell moments over velocity columns (k_cell's
-// work), one workgroup per cell.  Bound by memory (48^3 x 24^3 FP64: 24.7 -> 19.5 ms, about 6 TB/s with
-// what the L2 misses).  With F1 it also forms the cell macros and the next step's S1;
+// work), one workgroup per cell.  Bound by memory (48^3 x 24^3 FP64: 24.7 -> 19.7 ms, 5.6 TB/s with what
+// the L2 misses).  With F1 it also forms the cell macros and the next step's S1;
 // the new row of the first p.ntl tiles then stays in LDS and is written to HBM once.
 // Dynamic LDS: [velocity table (3 nax + 2) | axis table (LT nxi) | face tables of the fixed axes (NS la0) |
 // cell table of the fixed axes (la0) | incoming wall tables (NS nax) | row].
