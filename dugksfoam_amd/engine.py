@@ -246,19 +246,22 @@ class Engine:
         return bool(n.value)
 
     def blocks(self):
-        """Face kernel: (workgroup size, velocity iterations per thread, velocity blocks, padded Nv)."""
+        """Face kernel: (workgroup size, velocity iterations per thread, velocity blocks, padded Nv).
+        Column kernels: (64 lanes of a wave, iterations of a row over all waves, 1, padded Nv)."""
         v = [C.c_int32() for _ in range(4)]
         self._chk(load_library().dugks_get_launch(self._h, *[C.byref(x) for x in v]))
         return tuple(x.value for x in v)
 
     def cell_blocks(self):
-        """Cell kernel: (workgroup size, velocity iterations per thread, velocity blocks)."""
+        """Cell kernel: (workgroup size, velocity iterations per thread, velocity blocks); column
+        kernels as in blocks()."""
         v = [C.c_int32() for _ in range(3)]
         self._chk(load_library().dugks_get_cell_launch(self._h, *[C.byref(x) for x in v]))
         return tuple(x.value for x in v)
 
     def autotune(self, on: bool = True):
-        """Time the candidate work decompositions on the next steps and keep the fastest."""
+        """Time the candidate work decompositions on the next steps and keep the fastest; waits while
+        the column kernels run, which have one."""
         self._chk(load_library().dugks_set_autotune(self._h, 1 if on else 0))
 
     def autotune_steps_left(self) -> int:

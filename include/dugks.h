@@ -198,16 +198,18 @@ int dugks_set_graphs(dugks_engine* h, int32_t on);
  * with the shortest time of each.  The steps are
  * real steps of the simulation; the candidates differ only in how velocity sums are split,
  * i.e. in round-off.  The kernels over velocity columns (cells of up to 6 faces, 4 in 2-D, in
- * face-value mode) have one shape set by a rule: nothing is tuned there.
+ * face-value mode) have one shape set by a rule: nothing is tuned while they run, and the tuning
+ * waits for the first step of other kernels (dugks_set_face_values(h, 0)).
  * dugks_get_launch / dugks_get_cell_launch report the shapes in use. */
 int dugks_set_autotune(dugks_engine* h, int32_t on);
-/* Steps still to run before the tuning started by dugks_set_autotune ends (0 when idle). */
+/* Steps still to run before the tuning started by dugks_set_autotune ends (0 when idle or waiting). */
 int dugks_autotune_steps_left(dugks_engine* h, int32_t* steps);
 int dugks_get_cell_launch(dugks_engine* h, int32_t* nt, int32_t* nib, int32_t* n_blocks);
 
 /* Face-value mode (no reference counterpart): with it on, the face kernel stores every face
  * value it rebuilds ([face][velocity], storage precision) and the cell kernel reads them instead
- * of rebuilding them from gbar and its gradients.  FP64 results are bit-identical either way;
+ * of rebuilding them from gbar and its gradients.  FP64 results agree to the rounding of sums in
+ * another order (bit for bit with DUGKS_FACE_MFMA=0 and equal shapes);
  * with FP32 storage the face values are rounded to FP32 like the other stored rows.  Costs
  * n_faces x nv_padded x (4 or 8) bytes per carried distribution.  On by default when those
  * buffers take at most half of the free device memory at create. */
@@ -216,7 +218,9 @@ int dugks_get_face_values(dugks_engine* h, int32_t* on);
 
 /* Work decomposition of the face kernel (no reference counterpart; for measurement and
  * tuning): workgroup size, velocity iterations per thread in a block, number of
- * velocity blocks and the padded velocity count nt * nib * n_blocks.  NULL skips. */
+ * velocity blocks and the padded velocity count nt * nib * n_blocks.  With the kernels over velocity
+ * columns: the 64 lanes of a wave, the iterations of a row, which the one to four waves of a workgroup
+ * share tile by tile, and one block.  NULL skips. */
 int dugks_get_launch(dugks_engine* h, int32_t* nt, int32_t* nib, int32_t* n_blocks, int32_t* nv_padded);
 
 /* Complete resident state as an opaque byte image: resuming from it continues
