@@ -3538,9 +3538,14 @@ int dugks_create(const dugks_case *cs, dugks_engine **out)
         // memory; DUGKS_FACE_VALUES=0/1 in the environment forces it off/on
         const char *fv = std::getenv("DUGKS_FACE_VALUES");
         size_t fr = 0, tot = 0;
-        const size_t need = (size_t)h->nf * h->nvp * ts_size(h) * (h->has_h ? 2 : 1);
-        const bool fits = hipMemGetInfo(&fr, &tot) == hipSuccess && need <= fr / 2;
-        if (h->has_sym || (fv ? std::atoi(fv) != 0 : fits)) r = dugks_set_face_values(h, 1);
+        const bool known = hipMemGetInfo(&fr, &tot) == hipSuccess;
+        auto fits = [&] { return known && (size_t)h->nf * h->nvp * ts_size(h) * (h->has_h ? 2 : 1) <= fr / 2; };
+        if (h->line_ok && !fits()) {
+            // rows in columns have more padding, and build() could only estimate what would be left
+            r = set_rows(h, 0);
+            h->line_ok = 0;
+        }
+        if (!r && (h->has_sym || (fv ? std::atoi(fv) != 0 : fits()))) r = dugks_set_face_values(h, 1);
         const char *fl = std::getenv("DUGKS_FACE_PASS_LEGACY");
         h->face_pass_legacy = fl && std::atoi(fl) && !h->has_sym ? 1 : 0;
         // DUGKS_FACE_MFMA=0 keeps the FP64 face moments on the vector units

@@ -12,7 +12,7 @@ R, T0 = 208.0, 273.0
 
 
 def _hull(points, cell):
-    """The cell's faces as vertex lists, outward: for triangles and quads of the plane their edges, extruded."""
+    """The cell's faces as vertex lists, outward."""
     c = points[list(set(itertools.chain.from_iterable(cell)))].mean(axis=0)
     out = []
     for f in cell:

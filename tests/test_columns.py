@@ -112,7 +112,7 @@ def _box(dim, cells, name, nv, K=0, **sides):
 
 
 def _islands_2d(K, first):
-    """Triangles beside two quads, each cell on its own.  The first two triangles couple their vertical edges
+    """Four triangles and two quads, each cell on its own.  The first two triangles couple their vertical edges
     (a cyclic pair); the first face of the third is a far field; the fourth has walls only."""
     pts, cells = [], []
     shapes = [[(0, 0), (1, 0), (0, 1)], [(5, 0), (5, 1), (4, 1)], [(6, 0), (7, 0), (6, 1)], [(8, 0), (9, 0), (9, 1)],
